@@ -9,7 +9,8 @@
 // combinatorial rank used as FindStateIndex (:1431) in DH_INDEX_RANK mode:
 //   index(state) = dim - 1 - sum_{occupied j} T[j][n_j][s_j]
 // (n_j, s_j = number and index sum of the occupied orbitals <= j), split into a low-bit
-// table and a high-bit table so one lookup costs two table reads.
+// table and a high-bit table (which also holds dim - 1) so one lookup costs two table reads and a
+// subtraction.
 //
 // Spin1_2Chain (Spin/src/HilbertSpace/Spin1_2Chain.cc:113, :331) decides site 0 first and
 // keeps bits >= L at 1; its order is descending in the bit-reversed L-bit word, and
@@ -150,8 +151,9 @@ static int upload(dh_context* c, void** d, const void* h, size_t bytes) {
   return DH_OK;
 }
 
-// rank tables for a fermion sector (host): lo over the low `bits` orbitals, hi over the rest
-static void fermion_rank_tables(const SubsetCountTable& T, int nbrOrbitals, int N, int S, int bits,
+// rank tables for a fermion sector of dim states (host): lo over the low `bits` orbitals, hi (counted
+// down from dim - 1) over the rest
+static void fermion_rank_tables(const SubsetCountTable& T, int nbrOrbitals, int N, int S, int64_t dim, int bits,
                                 std::vector<uint32_t>& lo, std::vector<uint32_t>& hi) {
   lo.assign((size_t)1 << bits, 0);
   for (uint64_t l = 0; l < lo.size(); ++l) {
@@ -166,7 +168,7 @@ static void fermion_rank_tables(const SubsetCountTable& T, int nbrOrbitals, int 
     lo[l] = (uint32_t)acc;
   }
   int hb = nbrOrbitals - bits;
-  hi.assign((size_t)1 << hb, 0);
+  hi.assign((size_t)1 << hb, (uint32_t)(dim - 1));
   for (uint64_t h = 0; h < hi.size(); ++h) {
     int popH = __builtin_popcountll(h);
     int sumH = 0;
@@ -180,7 +182,7 @@ static void fermion_rank_tables(const SubsetCountTable& T, int nbrOrbitals, int 
       s += j;
       acc += T.at(j, n, s);
     }
-    hi[h] = (uint32_t)acc;
+    hi[h] = (uint32_t)(dim - 1 - acc);
   }
 }
 
@@ -234,7 +236,7 @@ extern "C" int dh_fermion_sphere_create(dh_context* c, dh_basis** out, int N, in
   // rank tables
   b->rankBits = dh_rank_split(nbrOrbitals);
   std::vector<uint32_t> lo, hi;
-  fermion_rank_tables(T, nbrOrbitals, N, S, b->rankBits, lo, hi);
+  fermion_rank_tables(T, nbrOrbitals, N, S, dim, b->rankBits, lo, hi);
   b->rankLoSize = (int64_t)lo.size();
   b->rankHiSize = (int64_t)hi.size();
   const std::vector<uint16_t> lo16 = dh_rank_lo16(lo);

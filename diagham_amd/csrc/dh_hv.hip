@@ -22,8 +22,8 @@
 
 // index lookup of the product kernels: where the rank tables live (both in LDS; the 16-bit low
 // table in LDS and the high table in global memory; both in global memory), and the row routine
-// (_X4: the created-pair loop unrolled four-wide; _FREE: only the free created pairs,
-// dh_sphere_row_free)
+// (_X4: the created-pair loop unrolled four-wide; _FREE: only the set bits of the mask
+// of free created pairs, dh_sphere_row)
 enum {
   MODE_BSEARCH = 0,
   MODE_RANK_LDS = 1,
@@ -129,7 +129,8 @@ __device__ __forceinline__ int64_t sphere_find(const SphereArgs& a, uint64_t tgt
 // so the row routine runs on 32-bit state words and 32-bit indices (used for k <= 2); 2 = 64-bit
 // state words with 32-bit indices (fewer than 2^31 states: the rank, its clamp and the gather
 // offset in 32-bit arithmetic); 0 = 64-bit words and indices.
-template <int K, int LPR, int MODE, int WORDS>
+// TRI: the factor matrices are triangles (dh_pack_sphere_factors).
+template <int K, int LPR, int MODE, int WORDS, bool TRI>
 __global__ void __launch_bounds__(1024) sphere_hv_kernel(SphereArgs a, const double* __restrict__ x,
                                                          double* __restrict__ y, int add, int64_t first,
                                                          int64_t count) {
@@ -163,35 +164,29 @@ __global__ void __launch_bounds__(1024) sphere_hv_kernel(SphereArgs a, const dou
       const uint32_t last = (uint32_t)a.dim - 1u, mask = (1u << a.rankBits) - 1u;
       const int bits = a.rankBits;
       // clamped so that a target outside the space can never address outside the vectors
-      auto find = [&](uint32_t t) -> uint32_t { return min(last - loAt(t & mask) - sHi[t >> bits], last); };
-      if constexpr (ROW == ROW_FREE)
-        dh_sphere_row_free<K, LPR>((uint32_t)s, a.nbrOrbitals, sF, sBase, lane, find, x, acc);
-      else if constexpr (ROW == ROW_X4)
-        dh_sphere_row_x4<K, LPR>((uint32_t)s, a.nbrOrbitals, sF, sBase, lane, find, x, acc);
+      auto find = [&](uint32_t t) -> uint32_t { return min(dh_word(sHi, t >> bits) - loAt(t & mask), last); };
+      if constexpr (ROW == ROW_X4)
+        dh_sphere_row_x4<K, LPR, TRI>((uint32_t)s, a.nbrOrbitals, sF, sBase, lane, find, x, (uint32_t)row, acc);
       else
-        dh_sphere_row<K, LPR>((uint32_t)s, a.nbrOrbitals, sF, sBase, lane, find, x, acc);
+        dh_sphere_row<K, LPR, ROW == ROW_FREE, TRI>((uint32_t)s, a.nbrOrbitals, sF, sBase, lane, find, x, (uint32_t)row, acc);
     } else if constexpr (WORDS == 2 && BASE != MODE_BSEARCH) {
       // rankBits = ceil(orbitals / 2) <= 32, so t >> bits fits 32 bits
       const uint32_t last = (uint32_t)a.dim - 1u;
       const uint32_t mask = a.rankBits >= 32 ? 0xffffffffu : (1u << a.rankBits) - 1u;
       const int bits = a.rankBits;
       auto find = [&](uint64_t t) -> uint32_t {
-        return min(last - loAt((uint32_t)t & mask) - sHi[(uint32_t)(t >> bits)], last);
+        return min(dh_word(sHi, (uint32_t)(t >> bits)) - loAt((uint32_t)t & mask), last);
       };
-      if constexpr (ROW == ROW_FREE)
-        dh_sphere_row_free<K, LPR>(s, a.nbrOrbitals, sF, sBase, lane, find, x, acc);
-      else if constexpr (ROW == ROW_X4)
-        dh_sphere_row_x4<K, LPR>(s, a.nbrOrbitals, sF, sBase, lane, find, x, acc);
+      if constexpr (ROW == ROW_X4)
+        dh_sphere_row_x4<K, LPR, TRI>(s, a.nbrOrbitals, sF, sBase, lane, find, x, (uint32_t)row, acc);
       else
-        dh_sphere_row<K, LPR>(s, a.nbrOrbitals, sF, sBase, lane, find, x, acc);
+        dh_sphere_row<K, LPR, ROW == ROW_FREE, TRI>(s, a.nbrOrbitals, sF, sBase, lane, find, x, (uint32_t)row, acc);
     } else {
       auto find = [&](uint64_t t) -> int64_t { return sphere_find<BASE>(a, t, sLut, sLo, sHi, sLo16); };
-      if constexpr (ROW == ROW_FREE)
-        dh_sphere_row_free<K, LPR>(s, a.nbrOrbitals, sF, sBase, lane, find, x, acc);
-      else if constexpr (ROW == ROW_X4)
-        dh_sphere_row_x4<K, LPR>(s, a.nbrOrbitals, sF, sBase, lane, find, x, acc);
+      if constexpr (ROW == ROW_X4)
+        dh_sphere_row_x4<K, LPR, TRI>(s, a.nbrOrbitals, sF, sBase, lane, find, x, row, acc);
       else
-        dh_sphere_row<K, LPR>(s, a.nbrOrbitals, sF, sBase, lane, find, x, acc);
+        dh_sphere_row<K, LPR, ROW == ROW_FREE, TRI>(s, a.nbrOrbitals, sF, sBase, lane, find, x, row, acc);
     }
     if constexpr (LPR > 1) {
 #pragma unroll
@@ -485,8 +480,10 @@ static int sphere_launch(dh_hamiltonian* h, int bs, const double* x, double* y, 
   const bool s32 = K <= 2 && idx32 && h->basis->nbrOrbitals <= 32;
   constexpr int W1 = (K <= 2 && MODE != MODE_BSEARCH) ? 1 : 0;
   constexpr int W2 = MODE != MODE_BSEARCH ? 2 : 0;
-  auto kern = s32 ? sphere_hv_kernel<K, LPR, MODE, W1>
-                  : (idx32 ? sphere_hv_kernel<K, LPR, MODE, W2> : sphere_hv_kernel<K, LPR, MODE, 0>);
+  auto kern = h->triangles ? (s32 ? sphere_hv_kernel<K, LPR, MODE, W1, true>
+                                  : (idx32 ? sphere_hv_kernel<K, LPR, MODE, W2, true> : sphere_hv_kernel<K, LPR, MODE, 0, true>))
+                           : (s32 ? sphere_hv_kernel<K, LPR, MODE, W1, false>
+                                  : (idx32 ? sphere_hv_kernel<K, LPR, MODE, W2, false> : sphere_hv_kernel<K, LPR, MODE, 0, false>));
   if (lds > 64 * 1024) DH_HIP(c, hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   int64_t rowsPerBlock = bs / LPR;
   dim3 grid;
@@ -773,7 +770,8 @@ extern "C" int dh_sphere_hamiltonian_create(dh_context* c, dh_hamiltonian** out,
     return dh_fail(c, DH_E_ARG, "nbr_factors does not match the factor layout");
   std::vector<double> packed;
   std::vector<int> sumBase;
-  int rc = dh_pack_factors_checked(c, nOrb, factors, pairOffset, packed, sumBase);
+  bool triangles;
+  int rc = dh_pack_factors_checked(c, nOrb, factors, pairOffset, packed, sumBase, triangles);
   if (rc) return rc;
   dh_hamiltonian* h = new dh_hamiltonian();
   h->ctx = c;
@@ -783,6 +781,7 @@ extern "C" int dh_sphere_hamiltonian_create(dh_context* c, dh_hamiltonian** out,
   h->nbrPairs = nPairs;
   h->nbrPackedFactors = (int)packed.size();
   h->nbrPairSums = (int)sumBase.size();
+  h->triangles = triangles;
   if ((rc = dh_alloc(c, (void**)&h->d_factors, sizeof(double) * std::max(nbrFactors, 1))) ||
       (rc = dh_alloc(c, (void**)&h->d_pairOffset, sizeof(int) * (nPairs + 1))) ||
       (rc = dh_alloc(c, (void**)&h->d_packedFactors, sizeof(double) * std::max<size_t>(packed.size(), 1))) ||

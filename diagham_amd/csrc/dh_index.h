@@ -23,15 +23,20 @@ __device__ __forceinline__ int64_t dh_find_bsearch(uint64_t target, const int* _
   return lo;  // in [lut[key+1], lut[key]) for every target of the sector
 }
 
+// Entry i of a table of less than 2^30 words, by a 32-bit byte offset (one address instruction)
+__device__ __forceinline__ uint32_t dh_word(const uint32_t* __restrict__ table, uint32_t i) {
+  return *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(table) + (i << 2));
+}
+
 // Combinatorial rank of a fermion state in the descending basis of its sector (the low table in 32
 // bits, or its 16-bit copy).
 template <typename L>
 __device__ __forceinline__ int64_t dh_find_rank(uint64_t target, const L* __restrict__ lo,
                                                 const uint32_t* __restrict__ hi, int bits, int64_t dim) {
   uint32_t a = lo[target & ((1ull << bits) - 1)];
-  uint32_t b = hi[target >> bits];
+  uint32_t b = hi[target >> bits];  // dim - 1 less the states that the high orbitals put before
   // clamped so that a target outside the sector can never address outside the vectors
-  int64_t r = dim - 1 - (int64_t)a - (int64_t)b;
+  int64_t r = (int64_t)b - (int64_t)a;
   return r < 0 ? 0 : (r >= dim ? dim - 1 : r);
 }
 

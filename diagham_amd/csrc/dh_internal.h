@@ -99,7 +99,7 @@ struct dh_basis {
   // (of the ordering key) are >= v, v in [0, 2^lutBits]
   int lutBits = 0, lutShift = 0;
   int* d_lut = nullptr;
-  // combinatorial rank tables (fermions): index = dim - 1 - (lo[s & (2^rankBits-1)] + hi[s >> rankBits]);
+  // combinatorial rank tables (fermions): index = hi[s >> rankBits] - lo[s & (2^rankBits-1)];
   // d_rankLo16: the same low table in 16 bits (null when a value does not fit), for LDS staging
   int rankBits = 0;
   int64_t rankLoSize = 0, rankHiSize = 0;
@@ -121,8 +121,9 @@ struct dh_hamiltonian {
   int nbrFactors = 0, nbrPairs = 0;
   double* d_factors = nullptr;
   int* d_pairOffset = nullptr;  // [nbrPairs + 1]
-  // the same factors packed symmetric per pair sum (what the product kernels stage in LDS)
+  // the same factors packed per pair sum (what the product kernels stage in LDS)
   int nbrPackedFactors = 0, nbrPairSums = 0;
+  bool triangles = false;
   double* d_packedFactors = nullptr;
   int* d_sumBase = nullptr;  // [nbrPairSums]
   // adjoint channel split
@@ -174,7 +175,8 @@ struct dh_sector_set {
   uint32_t* d_rankHi = nullptr;
   uint16_t* d_rankLo16 = nullptr;  // the low table in 16 bits (null when a value does not fit)
   int64_t* d_offsets = nullptr;
-  // sphere factors (per-pair layout, and packed symmetric per pair sum)
+  // sphere factors (per-pair layout, and packed per pair sum)
+  bool triangles = false;
   double* d_factors = nullptr;
   int* d_pairOffset = nullptr;
   int nbrFactors = 0, nbrPairs = 0;
@@ -401,6 +403,14 @@ inline int dh_blocks_per_cu(const dh_context* c, Kern kern, int blockSize, size_
   return perCU;
 }
 
+// Raises a kernel's VGPR allocation to 64, which costs no occupancy (8 wavefronts per SIMD either way).
+// A 64-bit shift (v_lshlrev_b64, v_lshrrev_b64, v_ashrrev_i64) whose amount sits in the last allocated
+// VGPR, 8 n + 7, reads a wrong amount now and then on gfx950, as is known of gfx90a, where the compiler
+// avoids it: the nbody kernels with 56 registers and such a shift gave wrong rows in the wavefronts
+// that shared a SIMD, those with 50, 57 or 58 none.  For kernels that the check of the built code
+// (tests/test_isa_cpu.py) names.
+__device__ __forceinline__ void dh_pad_vgprs() { asm volatile("" ::: "v63"); }
+
 // XCD-aware block remap: MI355X hands consecutive workgroups to its 8 XCDs round robin;
 // remapping gives every XCD one contiguous range of blocks so neighbouring rows (whose
 // gather targets are close) share that XCD's L2.
@@ -414,31 +424,59 @@ __device__ __forceinline__ unsigned dh_xcd_block(unsigned b, unsigned n) {
   return start + i;
 }
 
-// Two-body factors on the sphere are symmetric, F(a -> b) = F(b -> a), between the pairs of one
-// orbital sum S = n1 + n2.  Pair (n1 > n2) of sum S has position n1 - lo(S), lo(S) = S/2 + 1, and
-// the factor between positions i and j (i <= j) is packed at base[S] + j (j + 1) / 2 + i.  This
-// halves the table the product kernels stage in LDS.  Input: the per-pair layout (pair
-// a = n1 (n1 - 1) / 2 + n2, created m3 from lo(S): factors[pairOffset[a] + m3 - lo(S)]).
+// Two-body factors on the sphere as the product kernels stage them in LDS.  Pair (n1 > n2) of orbital
+// sum S = n1 + n2 has position n1 - lo(S), lo(S) = S/2 + 1.  The factors are symmetric, F(a -> b) =
+// F(b -> a).  Where they do not change either, apart from the diagonal ones F(a -> a), under the
+// reflection m -> nbrOrbitals - 1 - m, the sums S and 2 (nbrOrbitals - 1) - S have the same matrix,
+// position for position: then the table holds the diagonal factors by pair a = n1 (n1 - 1) / 2 + n2,
+// followed by one whole matrix (row i at i * np) for both sums, and a factor is one offset away.  Other
+// tables, and those of more than 100 KiB, keep one triangle per sum, j (j + 1) / 2 + i for i <= j, with
+// eight more instructions per factor.  An entry of base packs where the sum's matrix starts and its
+// number of pairs.  Input: the per-pair layout (pair a, created m3 from lo(S):
+// factors[pairOffset[a] + m3 - lo(S)]).
+constexpr int DH_SUM_BASE_BITS = 24;
+constexpr int DH_SUM_BASE_MASK = (1 << DH_SUM_BASE_BITS) - 1;
+
 inline void dh_pack_sphere_factors(int nbrOrbitals, const double* factors, const int* pairOffset,
-                                   std::vector<double>& packed, std::vector<int>& base) {
-  const int nbrSums = 2 * nbrOrbitals - 1;
+                                   std::vector<double>& packed, std::vector<int>& base, bool& triangles) {
+  const int nbrSums = 2 * nbrOrbitals - 1, centre = nbrOrbitals - 1, nbrPairs = nbrOrbitals * (nbrOrbitals - 1) / 2;
+  auto pairs = [&](int S) { return std::max(0, std::min(S, centre) - S / 2); };
+  auto at = [&](int S, int i, int j) {
+    const int n1 = S / 2 + 1 + i, n2 = S - n1;
+    return factors[pairOffset[n1 * (n1 - 1) / 2 + n2] + j];
+  };
+  size_t squares = nbrPairs;
+  for (int S = 0; S <= centre; ++S) squares += (size_t)pairs(S) * pairs(S);
+  triangles = squares * sizeof(double) > 100 * 1024;
+  for (int S = 0; S < centre; ++S)
+    for (int i = 0; i < pairs(S); ++i)
+      for (int j = 0; j < pairs(S); ++j)
+        if (i != j && at(S, i, j) != at(2 * centre - S, i, j)) triangles = true;
   packed.clear();
+  if (!triangles) {
+    packed.resize(nbrPairs);
+    for (int S = 0; S < nbrSums; ++S)
+      for (int i = 0; i < pairs(S); ++i) {
+        const int n1 = S / 2 + 1 + i;
+        packed[n1 * (n1 - 1) / 2 + S - n1] = at(S, i, i);
+      }
+  }
   base.assign(nbrSums, 0);
   for (int S = 0; S < nbrSums; ++S) {
-    base[S] = (int)packed.size();
-    const int lo = S / 2 + 1, hi = std::min(S, nbrOrbitals - 1);
-    for (int j = 0; lo + j <= hi; ++j)
-      for (int i = 0; i <= j; ++i) {
-        const int n1 = lo + i, n2 = S - n1;
-        packed.push_back(factors[pairOffset[n1 * (n1 - 1) / 2 + n2] + j]);
-      }
+    if (!triangles && S > centre) {
+      base[S] = base[2 * centre - S];
+      continue;
+    }
+    base[S] = (int)packed.size() | (pairs(S) << DH_SUM_BASE_BITS);
+    for (int j = 0; j < pairs(S); ++j)
+      for (int i = 0; i < (triangles ? j + 1 : pairs(S)); ++i) packed.push_back(triangles ? at(S, i, j) : at(S, j, i));
   }
 }
 
-// packs, and refuses factor tables that are not symmetric (the products read one triangle)
+// packs, and refuses factor tables that are not symmetric
 inline int dh_pack_factors_checked(dh_context* c, int nbrOrbitals, const double* factors, const int* pairOffset,
-                                   std::vector<double>& packed, std::vector<int>& base) {
-  dh_pack_sphere_factors(nbrOrbitals, factors, pairOffset, packed, base);
+                                   std::vector<double>& packed, std::vector<int>& base, bool& triangles) {
+  dh_pack_sphere_factors(nbrOrbitals, factors, pairOffset, packed, base, triangles);
   double scale = 0.0, asym = 0.0;
   for (int S = 0; S < 2 * nbrOrbitals - 1; ++S) {
     const int lo = S / 2 + 1, hi = std::min(S, nbrOrbitals - 1);
@@ -456,10 +494,6 @@ inline int dh_pack_factors_checked(dh_context* c, int nbrOrbitals, const double*
   return DH_OK;
 }
 
-__host__ __device__ __forceinline__ int dh_packed_index(int i, int j) {
-  return i <= j ? ((j * (j + 1)) >> 1) + i : ((i * (i + 1)) >> 1) + j;
-}
-
 // binomial C(n, k) for the host, 64-bit
 inline uint64_t dh_binom_host(int n, int k) {
   if (k < 0 || k > n) return 0;
@@ -468,7 +502,7 @@ inline uint64_t dh_binom_host(int n, int k) {
   return r;
 }
 
-// Low-table width of the combinatorial rank (index = dim - 1 - lo[low bits] - hi[high bits]).  The
+// Low-table width of the combinatorial rank (index = hi[high bits] - lo[low bits]).  The
 // low table counts patterns of the low orbitals with the same particle number and momentum, so its
 // values stay below C(bits, bits / 2) and fit 16 bits: at 14 bits it is 32 KiB and is staged in LDS
 // by the product kernels.  Up to 28 orbitals the split is even; from 29 to 34 orbitals the low part

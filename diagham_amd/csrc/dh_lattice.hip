@@ -142,6 +142,8 @@ extern "C" int dh_momentum_sector_set_create(dh_context* c, dh_sector_set** out,
       int popH = __builtin_popcountll(h), clsH = 0;
       for (uint64_t r = h; r; r &= r - 1) clsH = cl.add(clsH, S->rankBits + __builtin_ctzll(r));
       int n = N - popH;
+      const int64_t last = S->offsets[sec + 1] - S->offsets[sec] - 1;
+      hi[(size_t)sec * S->hiSize + h] = (uint32_t)last;
       if (n < 0) continue;
       int cc = cl.sub(target[sec], clsH);
       int64_t acc = 0;
@@ -151,7 +153,7 @@ extern "C" int dh_momentum_sector_set_create(dh_context* c, dh_sector_set** out,
         cc = cl.add(cc, j);
         acc += Tat(j, n, cc);
       }
-      hi[(size_t)sec * S->hiSize + h] = (uint32_t)acc;
+      hi[(size_t)sec * S->hiSize + h] = (uint32_t)(last - acc);
     }
   });
   const std::vector<uint16_t> lo16 = dh_rank_lo16(lo);

@@ -115,6 +115,8 @@ extern "C" int dh_sector_set_create(dh_context* c, dh_sector_set** out, int N, i
       int popH = __builtin_popcountll(h), sumH = 0;
       for (uint64_t r = h; r; r &= r - 1) sumH += S->rankBits + __builtin_ctzll(r);
       int n = N - popH, s = S->orbitalSum[sec] - sumH;
+      const int64_t last = S->offsets[sec + 1] - S->offsets[sec] - 1;
+      hi[(size_t)sec * S->hiSize + h] = (uint32_t)last;
       if (n < 0 || s < 0) continue;
       int64_t acc = 0;
       for (uint64_t r = h; r; r &= r - 1) {
@@ -123,7 +125,7 @@ extern "C" int dh_sector_set_create(dh_context* c, dh_sector_set** out, int N, i
         s += j;
         acc += Tat(j, n, s);
       }
-      hi[(size_t)sec * S->hiSize + h] = (uint32_t)acc;
+      hi[(size_t)sec * S->hiSize + h] = (uint32_t)(last - acc);
     }
   });
   const std::vector<uint16_t> lo16 = dh_rank_lo16(lo);
@@ -205,7 +207,8 @@ extern "C" int dh_sector_set_factors(dh_sector_set* S, const double* factors, co
   if (pairOffset[nPairs] != expect || nbrFactors != expect) return dh_fail(c, DH_E_ARG, "nbr_factors layout");
   std::vector<double> packed;
   std::vector<int> sumBase;
-  int rc = dh_pack_factors_checked(c, nOrb, factors, pairOffset, packed, sumBase);
+  bool triangles;
+  int rc = dh_pack_factors_checked(c, nOrb, factors, pairOffset, packed, sumBase, triangles);
   if (rc) return rc;
   hipStreamSynchronize(c->stream);
   for (void** p : {(void**)&S->d_factors, (void**)&S->d_pairOffset, (void**)&S->d_packedFactors, (void**)&S->d_sumBase}) {
@@ -228,6 +231,7 @@ extern "C" int dh_sector_set_factors(dh_sector_set* S, const double* factors, co
   S->nbrPairs = nPairs;
   S->nbrPackedFactors = (int)packed.size();
   S->nbrPairSums = (int)sumBase.size();
+  S->triangles = triangles;
   S->shift = shift;
   return DH_OK;
 }
@@ -328,8 +332,9 @@ __device__ __forceinline__ int tile_sector(const int64_t* sPrefix, int nActive, 
 // S32: the orbitals fit a 32-bit word, so the row routine runs on 32-bit state words (used for
 // k <= 2).  Every sector has fewer than 2^31 states (the set refuses larger ones), so indices are
 // 32-bit in both forms.
-// FREE: the created pairs come from the free-pair masks (dh_sphere_row_free).
-template <int K, int LPR, bool LO_LDS, bool S32, bool FREE>
+// FREE: the created pairs come from the set bits of the free-pair masks (dh_sphere_row).
+// TRI: the factor matrices are triangles (dh_pack_sphere_factors).
+template <int K, int LPR, bool LO_LDS, bool S32, bool FREE, bool TRI>
 __global__ void __launch_bounds__(1024) sectors_hv_kernel(SectorsArgs a, const double* __restrict__ x,
                                                           double* __restrict__ y, int add) {
   extern __shared__ double smem[];
@@ -370,23 +375,19 @@ __global__ void __launch_bounds__(1024) sectors_hv_kernel(SectorsArgs a, const d
       const uint32_t last = (uint32_t)dim - 1u, mask = (1u << a.rankBits) - 1u;
       const int bits = a.rankBits;
       // clamped so that a target outside the sector can never address outside the vectors
-      auto find = [&](uint32_t t) -> uint32_t { return min(last - loAt(t & mask) - hi[t >> bits], last); };
-      if constexpr (FREE)
-        dh_sphere_row_free<K, LPR>((uint32_t)s, a.nbrOrbitals, sF, sBase, lane, find, x + off * K, acc);
-      else
-        dh_sphere_row<K, LPR>((uint32_t)s, a.nbrOrbitals, sF, sBase, lane, find, x + off * K, acc);
+      auto find = [&](uint32_t t) -> uint32_t { return min(dh_word(hi, t >> bits) - loAt(t & mask), last); };
+      dh_sphere_row<K, LPR, FREE, TRI>((uint32_t)s, a.nbrOrbitals, sF, sBase, lane, find, x + off * K,
+                                       (uint32_t)(g - off), acc);
     } else {
       // rankBits = ceil(orbitals / 2) <= 32, so t >> bits fits 32 bits
       const uint32_t last = (uint32_t)dim - 1u;
       const uint32_t mask = a.rankBits >= 32 ? 0xffffffffu : (1u << a.rankBits) - 1u;
       const int bits = a.rankBits;
       auto find = [&](uint64_t t) -> uint32_t {
-        return min(last - loAt((uint32_t)t & mask) - hi[(uint32_t)(t >> bits)], last);
+        return min(dh_word(hi, (uint32_t)(t >> bits)) - loAt((uint32_t)t & mask), last);
       };
-      if constexpr (FREE)
-        dh_sphere_row_free<K, LPR>(s, a.nbrOrbitals, sF, sBase, lane, find, x + off * K, acc);
-      else
-        dh_sphere_row<K, LPR>(s, a.nbrOrbitals, sF, sBase, lane, find, x + off * K, acc);
+      dh_sphere_row<K, LPR, FREE, TRI>(s, a.nbrOrbitals, sF, sBase, lane, find, x + off * K,
+                                       (uint32_t)(g - off), acc);
     }
     if constexpr (LPR > 1) {
 #pragma unroll
@@ -434,9 +435,9 @@ static int sectors_hv_launch(dh_sector_set* S, const double* x, double* y, int a
   if (rc) return rc;
   if (tiles == 0) return DH_OK;
   size_t base = ((size_t)S->nbrPackedFactors * 8 + (size_t)S->nbrPairSums * 4 + 7) / 8 * 8 + 8 * (2 * na + 1);
-  // the 16-bit low table in LDS when it exists and the workgroup's tables stay within 64 KiB
+  // the 16-bit low table in LDS when it exists and two workgroups' tables fit a CU's 160 KiB
   size_t withLo = base + 2 * S->loSize;
-  bool loLds = S->d_rankLo16 && withLo <= 64 * 1024;
+  bool loLds = S->d_rankLo16 && withLo <= 79 * 1024;
   size_t lds = loLds ? withLo : base;
   if (lds > 160 * 1024) return dh_fail(c, DH_E_RANGE, "staged tables exceed LDS");
   SectorsArgs a = sectors_args(S, na, tiles);
@@ -455,18 +456,17 @@ static int sectors_hv_launch(dh_sector_set* S, const double* x, double* y, int a
   const bool s32 = K <= 2 && S->nbrOrbitals <= 32;
   // DH_INDEX_RANK: the free-pair masks for k <= 2, the range loop for k > 2 (the faster per k on
   // MI355X, as for a single space)
-  if (S->rowMode == DH_INDEX_RANK_FREE || (S->rowMode == DH_INDEX_RANK && K <= 2)) {
-    if (loLds)
-      return s32 ? launch(sectors_hv_kernel<K, LPR, true, (K <= 2), true>)
-                 : launch(sectors_hv_kernel<K, LPR, true, false, true>);
-    return s32 ? launch(sectors_hv_kernel<K, LPR, false, (K <= 2), true>)
-               : launch(sectors_hv_kernel<K, LPR, false, false, true>);
-  }
-  if (loLds)
-    return s32 ? launch(sectors_hv_kernel<K, LPR, true, (K <= 2), false>)
-               : launch(sectors_hv_kernel<K, LPR, true, false, false>);
-  return s32 ? launch(sectors_hv_kernel<K, LPR, false, (K <= 2), false>)
-             : launch(sectors_hv_kernel<K, LPR, false, false, false>);
+  const bool freePairs = S->rowMode == DH_INDEX_RANK_FREE || (S->rowMode == DH_INDEX_RANK && K <= 2);
+  auto pick = [&](auto lo, auto tri) -> int {
+    constexpr bool LO = decltype(lo)::value, TRI = decltype(tri)::value;
+    if (freePairs)
+      return s32 ? launch(sectors_hv_kernel<K, LPR, LO, (K <= 2), true, TRI>)
+                 : launch(sectors_hv_kernel<K, LPR, LO, false, true, TRI>);
+    return s32 ? launch(sectors_hv_kernel<K, LPR, LO, (K <= 2), false, TRI>)
+               : launch(sectors_hv_kernel<K, LPR, LO, false, false, TRI>);
+  };
+  if (S->triangles) return loLds ? pick(std::true_type{}, std::true_type{}) : pick(std::false_type{}, std::true_type{});
+  return loLds ? pick(std::true_type{}, std::false_type{}) : pick(std::false_type{}, std::false_type{});
 }
 
 template <int K>

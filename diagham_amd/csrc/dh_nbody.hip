@@ -64,6 +64,7 @@ template <int K, int LPR>
 __global__ void __launch_bounds__(1024) nbody3_hv_kernel(NBodyArgs a, const double* __restrict__ x,
                                                          double* __restrict__ y, int add, int64_t first,
                                                          int64_t count) {
+  if constexpr (K <= 2) dh_pad_vgprs();
   uint64_t* sMask;
   int *sPos, *sOff;
   int64_t* sFOff;

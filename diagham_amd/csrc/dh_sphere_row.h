@@ -15,17 +15,23 @@ __device__ __forceinline__ int dh_ctz(uint32_t v) { return __builtin_ctz(v); }
 __device__ __forceinline__ int dh_popc(uint64_t v) { return __popcll(v); }
 __device__ __forceinline__ int dh_popc(uint32_t v) { return __popc(v); }
 
-// dh_packed_index with a 24-bit multiply (positions stay below 2^12): a full-rate multiply-add
-// instead of the quarter-rate 32-bit multiply
-__device__ __forceinline__ int dh_packed_index_dev(int i, int j) {
-  const unsigned mx = (unsigned)max(i, j), mn = (unsigned)min(i, j);
-  return (int)((__umul24(mx, mx + 1u) >> 1) + mn);
-}
-
-// c, negated when the parity p is odd: the sign bit flipped (the same double as -c)
-__device__ __forceinline__ double dh_negate_if(double c, int p) {
-  return __hiloint2double(__double2hiint(c) ^ (int)((unsigned)p << 31), __double2loint(c));
-}
+// Off-diagonal factors of annihilated pair i of one sum in LDS (dh_pack_sphere_factors): a square's row,
+// or one triangle.  The entry of sBase packs where the sum's table starts and its number of pairs.
+template <bool TRI>
+struct dh_row_factors {
+  const double* f;
+  int i;
+  __device__ __forceinline__ dh_row_factors(const double* sF, int entry, int i_) : i(i_) {
+    f = sF + (entry & DH_SUM_BASE_MASK);
+    if (!TRI) f += __mul24(i_, (int)((unsigned)entry >> DH_SUM_BASE_BITS));
+  }
+  __device__ __forceinline__ double operator()(int j) const {
+    if (!TRI) return f[j];
+    // a 24-bit multiply (positions stay below 2^12) instead of the quarter-rate 32-bit one
+    const unsigned mx = (unsigned)max(i, j), mn = (unsigned)min(i, j);
+    return f[(__umul24(mx, mx + 1u) >> 1) + mn];
+  }
+};
 
 template <int K, typename I>
 __device__ __forceinline__ void dh_gather_fma(double* acc, const double* __restrict__ x, I idx, double coef) {
@@ -43,46 +49,95 @@ __device__ __forceinline__ void dh_gather_fma(double* acc, const double* __restr
   }
 }
 
-// Two-body terms of row state s: for every occupied pair n1 > n2 (annihilated as a_n1 a_n2,
-// sign = parity of the occupied orbitals at and above each), every created pair m3 > m4 with
-// m3 + m4 = n1 + n2 (created a+_m3 a+_m4 on the intermediate state) whose orbitals are free.
-// Lane `lane` of the row's LPR lanes takes m3 = m3lo + lane, m3lo + lane + LPR, ...
-// Factors come packed symmetric per pair sum (sF, sBase: see dh_pack_sphere_factors).
-// Target indices come from `find(target)`; x is indexed relative to `xbase`.  Each term is one
-// gather.  For K <= 2 the multiply-add of a term is deferred to the next term, after that term's
-// index loads are issued: a term's gather and the next term's index loads are then in flight
-// together, instead of one after the other (the terms are still added in their order, so the sum
-// is the same to the bit).  Wider K keep one gather in flight per term: their registers would
-// lower the occupancy that hides the latency there.
-template <int K, int LPR, typename U, typename Find>
+__device__ __forceinline__ uint64_t dh_bitrev(uint64_t v) { return __builtin_bitreverse64(v); }
+__device__ __forceinline__ uint32_t dh_bitrev(uint32_t v) { return __builtin_bitreverse32(v); }
+
+// What a row state s tells about the pairs (m3 > m4) of one orbital sum S, as 32-bit masks over their
+// positions i = m3 - lo(S), m3 = lo(S) + i, m4 = m4hi(S) - i, lo(S) = S/2 + 1, m4hi(S) = (S - 1)/2
+// (at most 31 positions for 62 orbitals).
+//
+// free(S): both orbitals free in s.  Word f of the free orbitals, shifted so that m3 lands on bit i,
+// and f reversed, shifted so that m4 lands on bit i; both are zero beyond the orbitals.
+// sign(S): parity of the occupied orbitals in [m4, m3), from the prefix parities P (bit m: parity of
+// the occupied orbitals below m) in the same way.
+//
+// A term that annihilates pair a and creates pair b of the same sum, b != a: two pairs of one sum are
+// nested, m4 < n2 < n1 < m3 or n2 < m4 < m3 < n1, so they have no orbital in common, b has to be free
+// in s itself, and taking n1, n2 out of s changes the number of orbitals in [m4, m3) by 0 or 2.  Its
+// sign, popc(s >> n1) + popc(s >> n2) + popc(t >> m3) + popc(t >> m4), is thus
+// sign(S)[a] + sign(S)[b].  The term b = a is diagonal: -F(a, a).
+template <typename U>
+struct dh_row_masks {
+  static constexpr int W = 8 * sizeof(U);
+  U f, rf, par, rpar;
+  __device__ __forceinline__ dh_row_masks(U s, int nbrOrbitals) {
+    const U full = nbrOrbitals >= W ? ~U(0) : ((U(1) << nbrOrbitals) - U(1));
+    f = ~s & full;
+    rf = dh_bitrev(f);
+    par = s << 1;
+#pragma unroll
+    for (int o = 1; o < W; o <<= 1) par ^= par << o;
+    rpar = dh_bitrev(par);
+  }
+  __device__ __forceinline__ uint32_t free(int m3lo, int m4hi) const {
+    return (uint32_t)(f >> m3lo) & (uint32_t)(rf >> (W - 1 - m4hi));
+  }
+  __device__ __forceinline__ uint32_t sign(int m3lo, int m4hi) const {
+    return (uint32_t)(par >> m3lo) ^ (uint32_t)(rpar >> (W - 1 - m4hi));
+  }
+};
+
+// the factor c with the sign that bit 31 - c of the position mask q gives its position
+__device__ __forceinline__ double dh_negate_by(double c, uint32_t signAtBit31) {
+  return __hiloint2double(__double2hiint(c) ^ (int)(signAtBit31 & 0x80000000u), __double2loint(c));
+}
+
+// Two-body terms of row state s: for every occupied pair n1 > n2 (annihilated) and every other pair
+// m3 > m4 of the same orbital sum that is free in s (created), one gather; the diagonal terms are
+// summed into one coefficient of x[self].  FREE walks the set bits of the free mask; otherwise every
+// position is tried against it (fewer registers).  Positions run from the highest down, and lane
+// `lane` of the row's LPR lanes takes every LPR-th (free) one.  Target indices come from
+// `find(target)`; x is indexed relative to `xbase`.
+//
+// A term costs 23 vector instructions on 32-bit and 28 on 64-bit words (36 and 46 before the masks over
+// positions, the square factor rows, and the diagonal terms apart), which leaves the gathers as the
+// bound: N=12 2S=33 Lz=0, k = 1, 5.6 -> 4.5 ms with the vector units busy 60 % of it (89 % before) and
+// one L1 access in every cycle, 27 per 64-lane gather.
+// For K <= 2 the multiply-add of a term is deferred to the next term, after that term's index loads
+// are issued: a term's gather and the next term's index loads are then in flight together (the terms
+// are still added in their order, so FREE and the range form agree to the bit at one lane per row).
+// Wider K keep one gather in flight per term: their registers would lower the occupancy that hides
+// the latency there.
+template <int K, int LPR, bool FREE, bool TRI, typename U, typename Find, typename I>
 __device__ __forceinline__ void dh_sphere_row(U s, int nbrOrbitals, const double* __restrict__ sF,
                                               const int* __restrict__ sBase, int lane, Find find,
-                                              const double* __restrict__ xbase, double* acc) {
+                                              const double* __restrict__ xbase, I self, double* acc) {
   constexpr bool PIPE = K <= 2;
   double pend[K];
-  double pendCoef = 0.0;
+  double pendCoef = 0.0, diag = 0.0;
 #pragma unroll
   for (int v = 0; v < K; ++v) pend[v] = 0.0;
+  const dh_row_masks<U> masks(s, nbrOrbitals);
   for (U r1 = s; r1; r1 &= r1 - 1) {
     const int n1 = dh_ctz(r1);
-    const int pc1 = dh_popc(s >> n1);
+    const double* diagRow = sF + __mul24(n1, n1 - 1) / 2;  // !TRI
+    double diag1 = 0.0;  // of this n1: two short sums round less than one long one
     for (U r2 = s & ((U(1) << n1) - U(1)); r2; r2 &= r2 - 1) {
       const int n2 = dh_ctz(r2);
-      const int sgnA = pc1 + dh_popc(s >> n2);
+      if (!TRI) diag1 += diagRow[n2];
+      const int sum = n1 + n2, m3lo = (sum >> 1) + 1, m4hi = (sum - 1) >> 1;
+      uint32_t pm = masks.free(m3lo, m4hi);
+      if (FREE && !TRI && !pm) continue;
       const U t = s ^ (U(1) << n1) ^ (U(1) << n2);
-      const int sum = n1 + n2;
-      const int m3lo = (sum >> 1) + 1;
-      const int m3hi = min(sum, nbrOrbitals - 1);
-      const double* fS = sF + sBase[sum];
-      const int i = n1 - m3lo;
-      for (int m3 = m3lo + lane; m3 <= m3hi; m3 += LPR) {
-        const int m4 = sum - m3;
-        const U cm = (U(1) << m3) | (U(1) << m4);
-        if (t & cm) continue;
-        const int sg = sgnA + dh_popc(t >> m4) + dh_popc(t >> m3);
-        const auto idx = find(t | cm);
-        double coef = fS[dh_packed_index_dev(i, m3 - m3lo)];
-        if (sg & 1) coef = -coef;
+      const int entry = sBase[sum], i = n1 - m3lo;
+      const dh_row_factors<TRI> F(sF, entry, i);
+      if (TRI) diag1 += F(i);
+      uint32_t q = masks.sign(m3lo, m4hi);
+      q ^= (uint32_t)-(int)((q >> i) & 1u);  // relative to the annihilated pair
+      // the created pair at position 31 - c (bit: its bit in a position mask), its sign in bit 31 of sg
+      auto term = [&](int c, uint32_t bit, uint32_t sg) {
+        const auto idx = find(t | (U(bit) << m3lo) | (U(1) << (m4hi - 31 + c)));
+        const double coef = dh_negate_by(F(31 - c), sg);
         if constexpr (PIPE) {
           // the previous term first, then this term's gather into the same registers (no copy,
           // so nothing waits for the gather before the next term's index loads)
@@ -95,13 +150,31 @@ __device__ __forceinline__ void dh_sphere_row(U s, int nbrOrbitals, const double
         } else {
           dh_gather_fma<K>(acc, xbase, idx, coef);
         }
+      };
+      if constexpr (FREE) {
+        if constexpr (LPR > 1)
+          for (int l = 0; l < lane && pm; ++l) pm ^= 0x80000000u >> __builtin_clz(pm);
+        while (pm) {
+          const int c = __builtin_clz(pm);
+          const uint32_t bit = 0x80000000u >> c;
+          pm ^= bit;
+#pragma unroll
+          for (int l = 1; l < LPR; ++l)  // past the other lanes' next ones
+            if (pm) pm ^= 0x80000000u >> __builtin_clz(pm);
+          term(c, bit, q << c);
+        }
+      } else {
+        for (int j = (int)((unsigned)entry >> DH_SUM_BASE_BITS) - 1 - lane; j >= 0; j -= LPR)
+          if ((pm >> j) & 1u) term(31 - j, 1u << j, q << (31 - j));
       }
     }
+    diag -= diag1;
   }
   if constexpr (PIPE) {
 #pragma unroll
     for (int v = 0; v < K; ++v) acc[v] = fma(pendCoef, pend[v], acc[v]);
   }
+  if (lane == 0) dh_gather_fma<K>(acc, xbase, self, diag);
 }
 
 // The same terms with the created-pair loop unrolled four-wide: a lane computes four targets
@@ -109,45 +182,44 @@ __device__ __forceinline__ void dh_sphere_row(U s, int nbrOrbitals, const double
 // coefficient), issues their index lookups together and then their four gathers, so four
 // dependent chains are in flight per lane.  `s` must be a state of the space (the padding
 // slots look it up).
-template <int K, int LPR, typename U, typename Find>
+template <int K, int LPR, bool TRI, typename U, typename Find, typename I>
 __device__ __forceinline__ void dh_sphere_row_x4(U s, int nbrOrbitals, const double* __restrict__ sF,
                                                  const int* __restrict__ sBase, int lane, Find find,
-                                                 const double* __restrict__ xbase, double* acc) {
+                                                 const double* __restrict__ xbase, I self, double* acc) {
+  const dh_row_masks<U> masks(s, nbrOrbitals);
+  double diag = 0.0;
   for (U r1 = s; r1; r1 &= r1 - 1) {
     const int n1 = dh_ctz(r1);
-    const int pc1 = dh_popc(s >> n1);
+    double diag1 = 0.0;
     for (U r2 = s & ((U(1) << n1) - U(1)); r2; r2 &= r2 - 1) {
       const int n2 = dh_ctz(r2);
-      const int sgnA = pc1 + dh_popc(s >> n2);
+      const int sum = n1 + n2, m3lo = (sum >> 1) + 1, m4hi = (sum - 1) >> 1;
       const U t = s ^ (U(1) << n1) ^ (U(1) << n2);
-      const int sum = n1 + n2;
-      const int m3lo = (sum >> 1) + 1;
-      const int m3hi = min(sum, nbrOrbitals - 1);
-      const double* fS = sF + sBase[sum];
-      const int i = n1 - m3lo;
-      for (int m3b = m3lo + lane; m3b <= m3hi; m3b += 4 * LPR) {
+      const int entry = sBase[sum], i = n1 - m3lo, np = (int)((unsigned)entry >> DH_SUM_BASE_BITS);
+      const dh_row_factors<TRI> F(sF, entry, i);
+      diag1 += TRI ? F(i) : sF[__mul24(n1, n1 - 1) / 2 + n2];
+      const uint32_t pm = masks.free(m3lo, m4hi);
+      uint32_t q = masks.sign(m3lo, m4hi);
+      q ^= (uint32_t)-(int)((q >> i) & 1u);
+      for (int jb = lane; jb < np; jb += 4 * LPR) {
         decltype(find(s)) idx[4];
         double coef[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          const int m3 = min(m3b + u * LPR, m3hi);  // clamped so that every shift stays in range
-          const int m4 = sum - m3;
-          const U cm = (U(1) << m3) | (U(1) << m4);
-          const bool ok = (m3b + u * LPR <= m3hi) && !(t & cm);
-          const int sg = sgnA + dh_popc(t >> m4) + dh_popc(t >> m3);
-          const double c = ok ? fS[dh_packed_index_dev(i, m3 - m3lo)] : 0.0;
-          coef[u] = (sg & 1) ? -c : c;
-          idx[u] = find(ok ? (t | cm) : s);
+          const int j = min(jb + u * LPR, np - 1);  // clamped so that every shift stays in range
+          const bool ok = (jb + u * LPR < np) && ((pm >> j) & 1u);
+          const double c = ok ? F(j) : 0.0;
+          coef[u] = dh_negate_by(c, q << (31 - j));
+          idx[u] = find(ok ? (t | (U(1) << (m3lo + j)) | (U(1) << (m4hi - j))) : s);
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) dh_gather_fma<K>(acc, xbase, idx[u], coef[u]);
       }
     }
+    diag -= diag1;
   }
+  if (lane == 0) dh_gather_fma<K>(acc, xbase, self, diag);
 }
-
-__device__ __forceinline__ uint64_t dh_bitrev(uint64_t v) { return __builtin_bitreverse64(v); }
-__device__ __forceinline__ uint32_t dh_bitrev(uint32_t v) { return __builtin_bitreverse32(v); }
 
 // Created pairs (m3 > m4, m3 + m4 = sum, both orbitals free in t) as a mask of their m3 bits:
 // bit m of f & (f mirrored about sum / 2) says that m and sum - m are both free.  The mirror of f
@@ -163,64 +235,4 @@ __device__ __forceinline__ U dh_free_pairs(U t, int nbrOrbitals, int sum, int m3
   const U hiMask = m3hi >= W - 1 ? ~U(0) : ((U(1) << (m3hi + 1)) - U(1));
   const U loMask = (U(1) << m3lo) - U(1);
   return f & mirror & hiMask & ~loMask;
-}
-
-// The terms of dh_sphere_row in the same order, with the created pairs taken from the mask of free
-// pairs of each annihilated pair (dh_free_pairs): no iteration is spent on a created pair with an
-// occupied orbital.  With LPR lanes on a row, lane l takes the free pairs l, l + LPR, ... of each
-// annihilated pair.  For K <= 2 a term's multiply-add waits for the next term's index loads, as in
-// dh_sphere_row, so the terms are added in the same order and with one lane per row the sum is
-// bitwise dh_sphere_row's.
-template <int K, int LPR, typename U, typename Find>
-__device__ __forceinline__ void dh_sphere_row_free(U s, int nbrOrbitals, const double* __restrict__ sF,
-                                                   const int* __restrict__ sBase, int lane, Find find,
-                                                   const double* __restrict__ xbase, double* acc) {
-  constexpr bool PIPE = K <= 2;
-  double pend[K];
-  double pendCoef = 0.0;
-#pragma unroll
-  for (int v = 0; v < K; ++v) pend[v] = 0.0;
-  // one created pair m3 > m4 = sum - m3 of the intermediate state t, with factor c
-  auto term = [&](U t, int sum, int sgnA, int m3, double c) {
-    const U b3 = U(1) << m3, b4 = U(1) << (sum - m3);
-    // the occupied orbitals of t at or above m4 and at or above m3 differ by those in [m4, m3)
-    const double coef = dh_negate_if(c, sgnA + dh_popc(t & (b3 - b4)));
-    const auto idx = find(t | b3 | b4);
-    if constexpr (PIPE) {
-      const double* xr = xbase + (size_t)idx * K;
-#pragma unroll
-      for (int v = 0; v < K; ++v) acc[v] = fma(pendCoef, pend[v], acc[v]);
-#pragma unroll
-      for (int v = 0; v < K; ++v) pend[v] = xr[v];
-      pendCoef = coef;
-    } else {
-      dh_gather_fma<K>(acc, xbase, idx, coef);
-    }
-  };
-  for (U r1 = s; r1; r1 &= r1 - 1) {
-    const int n1 = dh_ctz(r1);
-    const int pc1 = dh_popc(s >> n1);
-    for (U r2 = s & ((U(1) << n1) - U(1)); r2; r2 &= r2 - 1) {
-      const int n2 = dh_ctz(r2);
-      const int sgnA = pc1 + dh_popc(s >> n2);
-      const U t = s ^ (U(1) << n1) ^ (U(1) << n2);
-      const int sum = n1 + n2;
-      const int m3lo = (sum >> 1) + 1;
-      const double* fS = sF + sBase[sum];
-      const int i = n1 - m3lo;
-      U pm = dh_free_pairs(t, nbrOrbitals, sum, m3lo, min(sum, nbrOrbitals - 1));
-      if constexpr (LPR > 1)
-        for (int q = 0; q < lane; ++q) pm &= pm - 1;
-      while (pm) {
-        const int m3 = dh_ctz(pm);
-#pragma unroll
-        for (int q = 0; q < LPR; ++q) pm &= pm - 1;  // this term, then the other lanes' next ones
-        term(t, sum, sgnA, m3, fS[dh_packed_index_dev(i, m3 - m3lo)]);
-      }
-    }
-  }
-  if constexpr (PIPE) {
-#pragma unroll
-    for (int v = 0; v < K; ++v) acc[v] = fma(pendCoef, pend[v], acc[v]);
-  }
 }
