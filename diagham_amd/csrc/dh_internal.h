@@ -191,9 +191,9 @@ struct dh_sector_set {
   int64_t* d_sumFactorOff = nullptr;  // [nbrSums + 1] complex entries
   double* d_cfactors = nullptr;  // interleaved (re, im)
   int64_t nbrComplexFactors = 0;
-  // free-pair tables of a momentum set, per momentum sum j (see lattice_free_pairs): masks
+  // free-pair tables of a momentum set, per momentum sum j (see lattice_free_tables): masks
   // [3 j] = positions whose ky stays in its block / wraps / has the smaller orbital of its pair,
-  // shifts [2 j] = (kx rotation in bits, ky rotation), and per orbital m the pair (i2 << 8) | m2
+  // shifts [2 j] = (kx rotation in bits, ky rotation), and per orbital m the pair (i2 << 20) | m2
   uint64_t* d_freeMask = nullptr;
   int* d_freeShift = nullptr;
   int* d_partnerPos = nullptr;
@@ -206,7 +206,10 @@ struct dh_sector_set {
   double* d_phase = nullptr;   // per sector `modulo` (cos, sin) pairs
   int lutBits = 0, modulo = 1, stateShift = 0;
   int lanesPerRow = 1, blockSize = 256;
-  int rowMode = DH_INDEX_RANK;  // sphere sets: DH_INDEX_RANK or DH_INDEX_RANK_FREE row routine
+  // momentum sets: pick lanes per row and workgroup size per product from k and the rows (until
+  // dh_sector_set_launch is called)
+  bool autoLaunch = true;
+  int rowMode = DH_INDEX_RANK;  // DH_INDEX_RANK, _FREE or _RANGE row routine
   // segmented BLAS launch shape: persistent axpy workgroups per CU, dots rows per tile (0: auto)
   int axpyGroupsPerCU = 16;
   int64_t dotsRowsPerTile = 0;

@@ -198,7 +198,8 @@ extern "C" int dh_momentum_sector_set_create(dh_context* c, dh_sector_set** out,
 // ay = (Ny-1-jy) mod Ny bits inside every block.  Per sum: the rotation in bits ax Ny and ay, the
 // masks of the positions whose ky + ay stays below Ny (taken from g >> ay) or wraps (from
 // g << (Ny - ay)), the mask of the orbitals that are the smaller of their pair, and per orbital the
-// pair's position in the sum's list with its partner.
+// byte offset of the pair's complex factor in a row of the sum's matrix (16 times its position in the
+// sum's list) with its partner.
 static int lattice_free_tables(dh_sector_set* S, const std::vector<int>& info) {
   dh_context* c = S->ctx;
   const int nx = S->nbrSiteX, ny = S->nbrSiteY, N = S->nbrOrbitals, J = nx * ny;
@@ -220,7 +221,7 @@ static int lattice_free_tables(dh_sector_set* S, const std::vector<int>& info) {
         masks[3 * j + 2] |= 1ull << m;
         const int id = partner * (partner - 1) / 2 + m;
         if ((info[id] >> 16) != j) return dh_fail(c, DH_E_STATE, "momentum pair table inconsistent");
-        pp[(size_t)j * N + m] = ((info[id] & 0xffff) << 8) | partner;
+        pp[(size_t)j * N + m] = ((info[id] & 0xffff) << 20) | partner;
       }
     }
   }
@@ -308,7 +309,7 @@ extern "C" int dh_sector_set_lattice_factors(dh_sector_set* S, int nbrSums, cons
 struct LatticeArgs {
   const uint64_t* states;
   const int64_t* offsets;
-  int nbrOrbitals, nbrPairs, nbrSums, totalPairs;
+  int nbrOrbitals, nbrPairs, nbrSums, totalPairs, nbrFactors;
   int nbrSiteY;
   const uint64_t* freeMask;
   const int* freeShift;
@@ -341,33 +342,143 @@ __device__ __forceinline__ int lat_tile_sector(const int64_t* sPrefix, int nActi
   return lo;
 }
 
-// free created pairs of momentum sum j in t: bit m1 set when m1 and its partner are free and m1 is
-// the smaller of the two (tables of lattice_free_tables, in LDS)
-__device__ __forceinline__ uint64_t lattice_free_pairs(uint64_t t, int N, int ny, const uint64_t* __restrict__ mask,
-                                                       const int* __restrict__ shift, int j) {
-  const uint64_t full = N >= 64 ? ~0ull : ((1ull << N) - 1ull);
-  const uint64_t f = ~t & full;
-  const uint64_t R = __builtin_bitreverse64(f) >> (64 - N);
-  const int r = shift[2 * j], ay = shift[2 * j + 1];
-  const uint64_t g1 = r ? (((R >> r) | (R << (N - r))) & full) : R;
-  const uint64_t g = ((g1 >> ay) & mask[3 * j]) | ((g1 << (ny - ay)) & mask[3 * j + 1]);
-  return f & g & mask[3 * j + 2];
+// One row's words mirrored about a momentum sum j (tables of lattice_free_tables, in LDS): bit m1 of the
+// mirror is bit P_j(m1) of the word, given the word reversed within the N orbitals.
+template <typename U>
+__device__ __forceinline__ U lattice_mirror(U reversed, U full, int N, int ny, int rot, int ay, U stay, U wrap) {
+  const U g = rot ? (((reversed >> rot) | (reversed << (N - rot))) & full) : reversed;
+  return ((g >> ay) & stay) | ((g << ((ny - ay) & (8 * (int)sizeof(U) - 1))) & wrap);  // ay = 0: wrap is empty
 }
 
-// K complex vectors per row: x and y hold 2K doubles per row, (re, im) interleaved.  FREE: the
-// created pairs of each annihilated pair come from lattice_free_pairs (no iteration over a created
-// pair with an occupied orbital); otherwise every listed pair of the momentum sum is tried.
-template <int K, int LPR, bool LO_LDS, bool FREE>
+__device__ __forceinline__ uint64_t lat_bitrev(uint64_t v) { return __builtin_bitreverse64(v); }
+__device__ __forceinline__ uint32_t lat_bitrev(uint32_t v) { return __builtin_bitreverse32(v); }
+__device__ __forceinline__ int lat_ctz(uint64_t v) { return __builtin_ctzll(v); }
+__device__ __forceinline__ int lat_ctz(uint32_t v) { return __builtin_ctz(v); }
+__device__ __forceinline__ int lat_clz(uint64_t v) { return __builtin_clzll(v); }
+__device__ __forceinline__ int lat_clz(uint32_t v) { return __builtin_clz(v); }
+__device__ __forceinline__ double lat_flip(double v, uint32_t signAtBit31) {
+  return __hiloint2double(__double2hiint(v) ^ (int)(signAtBit31 & 0x80000000u), __double2loint(v));
+}
+
+struct LatticeTables {  // LDS
+  const int64_t* facOff;
+  const uint64_t* mask;
+  const double2* diag;  // by pair id
+  const int *info, *pairOff, *shift, *pp;
+};
+
+// The terms of row state s from free-pair masks.  Annihilated pair n1 < n2 of momentum sum j: two pairs
+// of one sum have no orbital in common, so every other pair of the sum that is free in s can be created,
+// one bit of pm each (bit m1, the smaller orbital), and the pair itself is the diagonal term -conj(F).
+// The sign of a created pair (m1, m2) on t is the parity of the occupied orbitals of t in [m1, m2): P(m1)
+// + P(m2) with the prefix parities P of t, those of s changed in (n1, n2]; q holds it at bit m1, with the
+// annihilated pair's (the same at n1) and the sign of the reordering taken in.  Bits run from the
+// highest; lane `lane` of LPR takes every LPR-th.  For K <= 2 a term's multiply-add waits for the next
+// term's index loads, so a gather and the next index loads are in flight together (in the same order).
+//
+// Bound by L1 accesses: a term gathers 16 bytes of x, a high rank table word and the factor, about 30 line
+// accesses each per wavefront.  With the factors in LDS the L1 has two thirds of them (41 M of 55 M cycles a
+// CU; 62 M of 74 M without).  32-bit words (up to 32 orbitals) take 30 vector instructions a term, 60 with a
+// free mask per intermediate state and popcounts on 64-bit words.  30 sectors of 10 fermions on 6 x 5 sites:
+// 46.4 ms so, 31.0 with these masks, 23.5 with the factors in LDS.
+template <int K, int LPR, typename U, typename Find>
+__device__ __forceinline__ void lattice_row_free(U s, int N, int ny, const LatticeTables& T,
+                                                 const double2* factors, int lane, Find find,
+                                                 const double* __restrict__ xs, uint32_t self, double* acc) {
+  constexpr int W = 8 * sizeof(U);
+  constexpr bool PIPE = K <= 2;
+  const U full = N >= W ? ~U(0) : ((U(1) << N) - U(1)), top = U(1) << (W - 1);
+  const U f = ~s & full, rf = lat_bitrev(f) >> (W - N);
+  U par = s << 1;
+#pragma unroll
+  for (int o = 1; o < W; o <<= 1) par ^= par << o;
+  par &= full;
+  double pre = 0.0, pim = 0.0, dr = 0.0, di = 0.0;
+  double2 px[K];
+#pragma unroll
+  for (int v = 0; v < K; ++v) px[v] = make_double2(0.0, 0.0);
+  auto add = [&](double cr, double ci, int v, double2 p) {
+    acc[2 * v] += cr * p.x - ci * p.y;
+    acc[2 * v + 1] += cr * p.y + ci * p.x;
+  };
+  for (U r2 = s; r2; r2 &= r2 - 1) {
+    const int n2 = lat_ctz(r2);  // higher annihilated orbital
+    const U below2 = (U(1) << n2) - U(1);
+    for (U r1 = s & below2; r1; r1 &= r1 - 1) {
+      const int n1 = lat_ctz(r1);  // lower annihilated orbital
+      const int id = __mul24(n2, n2 - 1) / 2 + n1;
+      const double2 fd = T.diag[id];
+      dr -= fd.x;
+      di += fd.y;
+      const int info = T.info[id], sum = info >> 16;
+      const int rot = T.shift[2 * sum], ay = T.shift[2 * sum + 1];
+      const U stay = (U)T.mask[3 * sum], wrap = (U)T.mask[3 * sum + 1], small = (U)T.mask[3 * sum + 2];
+      const U b1 = U(1) << n1;
+      const U t = s ^ b1 ^ (U(1) << n2);
+      U pm = f & lattice_mirror(rf, full, N, ny, rot, ay, stay, wrap) & small;
+      const U pt = par ^ ((below2 + below2 + U(1)) & ~(b1 + b1 - U(1)));  // orbitals in (n1, n2] flip
+      U q = pt ^ lattice_mirror((U)(lat_bitrev(pt) >> (W - N)), full, N, ny, rot, ay, stay, wrap);
+      q = (q & b1) ? q : ~q;
+      const int np = T.pairOff[sum + 1] - T.pairOff[sum];
+      const char* F = reinterpret_cast<const char*>(factors + ((int)T.facOff[sum] + __mul24(info & 0xffff, np)));
+      const int* pp = T.pp + sum * N + (W - 1);
+      if constexpr (LPR > 1)
+        for (int l = 0; l < lane && pm; ++l) pm ^= top >> lat_clz(pm);
+      while (pm) {
+        const int c = lat_clz(pm);
+        const U bit = top >> c;
+        pm ^= bit;
+#pragma unroll
+        for (int l = 1; l < LPR; ++l)  // past the other lanes' next ones
+          if (pm) pm ^= top >> lat_clz(pm);
+        const uint32_t e = (uint32_t)pp[-c];
+        const uint32_t idx = find(t | bit | (U(1) << (e & (W - 1))));
+        const double2 fe = *reinterpret_cast<const double2*>(F + (e >> 16));
+        const uint32_t sg = W == 64 ? (uint32_t)((uint64_t)(q << c) >> 32) : (uint32_t)(q << c);
+        const double cr = lat_flip(fe.x, sg), ci = lat_flip(fe.y, ~sg);  // conj(F), signed
+        const double* xr = xs + (size_t)idx * 2 * K;
+        if constexpr (PIPE) {
+#pragma unroll
+          for (int v = 0; v < K; ++v) add(pre, pim, v, px[v]);
+#pragma unroll
+          for (int v = 0; v < K; ++v) px[v] = *reinterpret_cast<const double2*>(xr + 2 * v);
+          pre = cr;
+          pim = ci;
+        } else {
+#pragma unroll
+          for (int v = 0; v < K; ++v) add(cr, ci, v, *reinterpret_cast<const double2*>(xr + 2 * v));
+        }
+      }
+    }
+  }
+  if constexpr (PIPE) {
+#pragma unroll
+    for (int v = 0; v < K; ++v) add(pre, pim, v, px[v]);
+  }
+  if (lane == 0) {
+    const double* xr = xs + (size_t)self * 2 * K;
+#pragma unroll
+    for (int v = 0; v < K; ++v) add(dr, di, v, *reinterpret_cast<const double2*>(xr + 2 * v));
+  }
+}
+
+// K complex vectors per row: x and y hold 2K doubles per row, (re, im) interleaved.  ROWS: 0, every
+// listed pair of the momentum sum is tried; 32 and 64, the free-pair masks (lattice_row_free) on words
+// of that many bits.
+template <int K, int LPR, bool LO_LDS, int ROWS, bool FAC_LDS>
 __global__ void __launch_bounds__(1024) lattice_hv_kernel(LatticeArgs a, const double* __restrict__ x,
                                                           double* __restrict__ y, int add) {
-  extern __shared__ int64_t smem64[];
-  int64_t* sWork = smem64;                                    // 2 nActive + 1
+  constexpr bool FREE = ROWS != 0;
+  extern __shared__ __align__(16) int64_t smem64[];
+  double2* sDiag = reinterpret_cast<double2*>(smem64);        // FREE: nbrPairs
+  double2* sFac = sDiag + (FREE ? a.nbrPairs : 0);            // FAC_LDS: nbrFactors
+  int64_t* sWork = reinterpret_cast<int64_t*>(sFac + (FAC_LDS ? a.nbrFactors : 0));  // 2 nActive + 1
   int64_t* sFacOff = sWork + 2 * a.nActive + 1;               // nbrSums + 1
   uint64_t* sMask = reinterpret_cast<uint64_t*>(sFacOff + a.nbrSums + 1);  // FREE: 3 nbrSums
   int* sInfo = reinterpret_cast<int*>(sMask + (FREE ? 3 * a.nbrSums : 0));  // nbrPairs
   int* sPairOff = sInfo + a.nbrPairs;                         // nbrSums + 1
-  int* sPairs = sPairOff + a.nbrSums + 1;                     // totalPairs
-  int* sShift = sPairs + a.totalPairs;                        // FREE: 2 nbrSums
+  int* sPairs = sPairOff + a.nbrSums + 1;                     // !FREE: totalPairs
+  int* sShift = sPairs + (FREE ? 0 : a.totalPairs);           // FREE: 2 nbrSums
   int* sPP = sShift + (FREE ? 2 * a.nbrSums : 0);             // FREE: nbrSums * nbrOrbitals
   // the low table: its 16-bit copy in LDS (LO_LDS), or the 32-bit table in global memory
   using LoT = typename std::conditional<LO_LDS, uint16_t, uint32_t>::type;
@@ -377,13 +488,24 @@ __global__ void __launch_bounds__(1024) lattice_hv_kernel(LatticeArgs a, const d
     sFacOff[i] = a.sumFactorOff[i];
     sPairOff[i] = a.sumPairOff[i];
   }
-  for (int i = threadIdx.x; i < a.nbrPairs; i += blockDim.x) sInfo[i] = a.pairInfo[i];
-  for (int i = threadIdx.x; i < a.totalPairs; i += blockDim.x) sPairs[i] = a.sumPairs[i];
+  for (int i = threadIdx.x; i < a.nbrPairs; i += blockDim.x) {
+    const int info = a.pairInfo[i];
+    sInfo[i] = info;
+    if constexpr (FREE) {
+      const int sum = info >> 16, i1 = info & 0xffff, np = a.sumPairOff[sum + 1] - a.sumPairOff[sum];
+      sDiag[i] = *reinterpret_cast<const double2*>(a.factors + 2 * (a.sumFactorOff[sum] + (int64_t)i1 * np + i1));
+    }
+  }
   if constexpr (FREE) {
     for (int i = threadIdx.x; i < 3 * a.nbrSums; i += blockDim.x) sMask[i] = a.freeMask[i];
     for (int i = threadIdx.x; i < 2 * a.nbrSums; i += blockDim.x) sShift[i] = a.freeShift[i];
     for (int i = threadIdx.x; i < a.nbrSums * a.nbrOrbitals; i += blockDim.x) sPP[i] = a.partnerPos[i];
+  } else {
+    for (int i = threadIdx.x; i < a.totalPairs; i += blockDim.x) sPairs[i] = a.sumPairs[i];
   }
+  if constexpr (FAC_LDS)
+    for (int i = threadIdx.x; i < a.nbrFactors; i += blockDim.x)
+      sFac[i] = reinterpret_cast<const double2*>(a.factors)[i];
   if constexpr (LO_LDS)
     for (int i = threadIdx.x; i < a.loSize; i += blockDim.x) sLo[i] = a.rankLo16[i];
   __syncthreads();
@@ -410,71 +532,20 @@ __global__ void __launch_bounds__(1024) lattice_hv_kernel(LatticeArgs a, const d
     for (int v = 0; v < 2 * K; ++v) acc[v] = 0.0;
     const double* xs = x + off * 2 * K;
     if constexpr (FREE) {
-      // every annihilated pair n1 < n2, then its free created pairs from the mask of lattice_free_pairs
-      // (lane `lane` of LPR takes every LPR-th of them); for K <= 2 a term's multiply-add waits for
-      // the next term's index loads, as in the list loop below, with the terms in the same order
-      constexpr bool PIPE = K <= 2;
-      double pre = 0.0, pim = 0.0;
-      double2 px[K];
-#pragma unroll
-      for (int v = 0; v < K; ++v) px[v] = make_double2(0.0, 0.0);
-      for (uint64_t r1 = s; r1; r1 &= r1 - 1) {
-        const int n1 = __builtin_ctzll(r1);  // lower annihilated orbital
-        for (uint64_t r2 = s & ~((2ull << n1) - 1ull); r2; r2 &= r2 - 1) {
-          const int n2 = __builtin_ctzll(r2);  // higher annihilated orbital
-          // AA(n1, n2): a_n2 first, then a_n1
-          const int sgnA = __popcll(s >> n2) + __popcll((s ^ (1ull << n2)) >> n1);
-          const uint64_t t = s ^ (1ull << n1) ^ (1ull << n2);
-          const int info = sInfo[(n2 * (n2 - 1)) / 2 + n1];
-          const int sum = info >> 16;
-          const int np = sPairOff[sum + 1] - sPairOff[sum];
-          const double* F = a.factors + 2 * (sFacOff[sum] + (int64_t)(info & 0xffff) * np);
-          const int* pp = sPP + sum * a.nbrOrbitals;
-          uint64_t pm = lattice_free_pairs(t, a.nbrOrbitals, a.nbrSiteY, sMask, sShift, sum);
-          if constexpr (LPR > 1)
-            for (int q = 0; q < lane; ++q) pm &= pm - 1;
-          while (pm) {
-            const int m1 = __builtin_ctzll(pm);
-#pragma unroll
-            for (int q = 0; q < LPR; ++q) pm &= pm - 1;  // this term, then the other lanes' next ones
-            const int pk = pp[m1];
-            const int m2 = pk & 0xff, i2 = pk >> 8;  // m1 < m2
-            const uint64_t c1 = 1ull << m1, c2 = 1ull << m2;
-            // AdAd(m1, m2), a+_m2 first, then a+_m1: popc(t >> m2) + popc((t | c2) >> m1) has the
-            // parity of 1 + the occupied orbitals of t in [m1, m2)
-            const int par = sgnA + 1 + __popcll(t & (c2 - c1));
-            const int64_t idx = dh_find_rank(t | c1 | c2, lo, hi, a.rankBits, dim);
-            const double2 f = *reinterpret_cast<const double2*>(F + 2 * i2);
-            const double cr = (par & 1) ? -f.x : f.x, ci = (par & 1) ? f.y : -f.y;  // conj(F), signed
-            const double* xr = xs + idx * 2 * K;
-            if constexpr (PIPE) {
-#pragma unroll
-              for (int v = 0; v < K; ++v) {
-                acc[2 * v] += pre * px[v].x - pim * px[v].y;
-                acc[2 * v + 1] += pre * px[v].y + pim * px[v].x;
-              }
-#pragma unroll
-              for (int v = 0; v < K; ++v) px[v] = *reinterpret_cast<const double2*>(xr + 2 * v);
-              pre = cr;
-              pim = ci;
-            } else {
-#pragma unroll
-              for (int v = 0; v < K; ++v) {
-                double2 p = *reinterpret_cast<const double2*>(xr + 2 * v);
-                acc[2 * v] += cr * p.x - ci * p.y;
-                acc[2 * v + 1] += cr * p.y + ci * p.x;
-              }
-            }
-          }
-        }
-      }
-      if constexpr (PIPE) {
-#pragma unroll
-        for (int v = 0; v < K; ++v) {
-          acc[2 * v] += pre * px[v].x - pim * px[v].y;
-          acc[2 * v + 1] += pre * px[v].y + pim * px[v].x;
-        }
-      }
+      using U = typename std::conditional<ROWS == 32, uint32_t, uint64_t>::type;
+      const LatticeTables T{sFacOff, sMask, sDiag, sInfo, sPairOff, sShift, sPP};
+      const uint32_t last = (uint32_t)dim - 1u, mask = (uint32_t)a.loSize - 1u;
+      const int bits = a.rankBits;
+      // clamped so that a target outside the sector can never address outside the vectors
+      auto find = [&](U t) -> uint32_t {
+        return min(dh_word(hi, (uint32_t)(t >> bits)) - lo[(uint32_t)t & mask], last);
+      };
+      const double2* fac;
+      if constexpr (FAC_LDS)
+        fac = sFac;
+      else
+        fac = reinterpret_cast<const double2*>(a.factors);
+      lattice_row_free<K, LPR, U>((U)s, a.nbrOrbitals, a.nbrSiteY, T, fac, lane, find, xs, (uint32_t)(g - off), acc);
     } else {
       // K <= 2: a term's multiply-add waits until the next term's index loads are issued, so the
       // gather of one term and the index loads of the next are in flight together (terms are still
@@ -552,10 +623,41 @@ __global__ void __launch_bounds__(1024) lattice_hv_kernel(LatticeArgs a, const d
   }
 }
 
+// Dynamic LDS of the lattice kernel for `na` active sectors: the tables of the row routine, with the
+// 16-bit low rank table, with that and every factor matrix.
+struct LatticeLds {
+  bool free;  // DH_INDEX_RANK: the free-pair masks
+  size_t tables, withLo, withFactors;
+  bool factorsFit;  // one workgroup of a CU can hold all of it (32-bit words only: 30 orbitals take 147 KiB)
+};
+
+static LatticeLds lattice_lds(const dh_sector_set* S, int na) {
+  LatticeLds l;
+  auto size = [&] {
+    const size_t bytes = 8 * (2 * (size_t)na + 1) + 8 * (size_t)(S->nbrSums + 1) + 4 * (size_t)S->nbrPairs +
+                         4 * (size_t)(S->nbrSums + 1) +
+                         (l.free ? 16 * (size_t)S->nbrPairs + 8 * 3 * (size_t)S->nbrSums + 4 * 2 * (size_t)S->nbrSums +
+                                       4 * (size_t)S->nbrSums * S->nbrOrbitals
+                                 : 4 * (size_t)S->nbrPairs);
+    return (bytes + 7) & ~size_t(7);
+  };
+  l.free = S->rowMode != DH_INDEX_RANK_RANGE && S->d_freeMask;
+  l.tables = size();
+  if (l.free && l.tables > 160 * 1024) {  // thousands of sectors: the pair lists take less
+    l.free = false;
+    l.tables = size();
+  }
+  l.withLo = l.tables + 2 * (size_t)S->loSize;
+  l.withFactors = l.withLo + 16 * (size_t)S->nbrComplexFactors;
+  l.factorsFit = l.free && S->d_rankLo16 && S->nbrOrbitals <= 32 && l.withFactors <= 160 * 1024;
+  return l;
+}
+
 template <int K, int LPR>
-static int lattice_launch(dh_sector_set* S, const double* x, double* y, int add, const unsigned char* active) {
+static int lattice_launch(dh_sector_set* S, int blockSize, const double* x, double* y, int add,
+                          const unsigned char* active) {
   dh_context* c = S->ctx;
-  int64_t rowsPerTile = S->blockSize / LPR;
+  int64_t rowsPerTile = blockSize / LPR;
   int na;
   int64_t tiles;
   int rc = dh_sectors_upload_work(S, active, rowsPerTile, &na, &tiles);
@@ -568,6 +670,7 @@ static int lattice_launch(dh_sector_set* S, const double* x, double* y, int add,
   a.nbrPairs = S->nbrPairs;
   a.nbrSums = S->nbrSums;
   a.totalPairs = S->nbrPairs;
+  a.nbrFactors = (int)S->nbrComplexFactors;
   a.pairInfo = S->d_pairInfo;
   a.sumPairOff = S->d_sumPairOff;
   a.sumPairs = S->d_sumPairs;
@@ -587,38 +690,59 @@ static int lattice_launch(dh_sector_set* S, const double* x, double* y, int add,
   a.freeMask = S->d_freeMask;
   a.freeShift = S->d_freeShift;
   a.partnerPos = S->d_partnerPos;
-  // DH_INDEX_RANK: the free-pair masks for one vector (35.7 against 40.3 ms for the 30 sectors of
-  // N=10 on 6 x 5 sites on MI355X), the pair list above (equal at k = 2, faster at k = 4)
-  const bool free = (S->rowMode == DH_INDEX_RANK_FREE || (S->rowMode == DH_INDEX_RANK && K == 1)) && S->d_freeMask;
-  size_t base = 8 * (2 * (size_t)na + 1) + 8 * (size_t)(S->nbrSums + 1) + 4 * (size_t)S->nbrPairs +
-                4 * (size_t)(S->nbrSums + 1) + 4 * (size_t)S->nbrPairs;
-  if (free) base += 8 * 3 * (size_t)S->nbrSums + 4 * 2 * (size_t)S->nbrSums + 4 * (size_t)S->nbrSums * S->nbrOrbitals;
-  base = (base + 7) & ~size_t(7);
-  size_t withLo = base + 2 * (size_t)S->loSize;
-  bool loLds = S->d_rankLo16 && withLo <= 64 * 1024;
-  size_t lds = loLds ? withLo : base;
+  const LatticeLds l = lattice_lds(S, na);
+  // the factors in LDS for a workgroup that fills its CU (16 wavefronts); smaller ones would leave it empty
+  const bool facLds = l.factorsFit && blockSize == 1024;
+  const bool loLds = S->d_rankLo16 && l.withLo <= 79 * 1024;  // two workgroups' tables in a CU's 160 KiB
+  const size_t lds = facLds ? l.withFactors : loLds ? l.withLo : l.tables;
   if (lds > 160 * 1024) return dh_fail(c, DH_E_RANGE, "staged tables exceed LDS");
   auto launch = [&](auto kern) -> int {
     if (lds > 64 * 1024)
       DH_HIP(c, hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    const int perCU = dh_blocks_per_cu(c, kern, S->blockSize, lds);
+    const int perCU = dh_blocks_per_cu(c, kern, blockSize, lds);
     int64_t grid = std::max<int64_t>(1, std::min<int64_t>(tiles, (int64_t)c->nbrCU * perCU));
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(S->blockSize), lds, c->stream, a, x, y, add);
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(blockSize), lds, c->stream, a, x, y, add);
     DH_HIP(c, hipGetLastError());
     return DH_OK;
   };
-  if (free) return loLds ? launch(lattice_hv_kernel<K, LPR, true, true>) : launch(lattice_hv_kernel<K, LPR, false, true>);
-  if (loLds) return launch(lattice_hv_kernel<K, LPR, true, false>);
-  return launch(lattice_hv_kernel<K, LPR, false, false>);
+  if (!l.free)
+    return loLds ? launch(lattice_hv_kernel<K, LPR, true, 0, false>) : launch(lattice_hv_kernel<K, LPR, false, 0, false>);
+  if (facLds) return launch(lattice_hv_kernel<K, LPR, true, 32, true>);
+  if (S->nbrOrbitals <= 32)
+    return loLds ? launch(lattice_hv_kernel<K, LPR, true, 32, false>)
+                 : launch(lattice_hv_kernel<K, LPR, false, 32, false>);
+  return loLds ? launch(lattice_hv_kernel<K, LPR, true, 64, false>)
+               : launch(lattice_hv_kernel<K, LPR, false, 64, false>);
+}
+
+// Lanes per row and workgroup size by rows per CU and k, times in us on MI355X.  Few rows: lanes for
+// wavefronts (8008 rows: 21.0 with 4 x 256, 25.5 with 1 x 256; k = 4: 24.7 with 8 x 256, 40.8).  Up to
+// 512 rows a CU 2 x 512 (53 k rows: 27.0 against 34.9).  Above, where the factors fit LDS, 1 x 1024
+// with them there (177 k rows 55.9 against 63.6 at 1 x 256 and 61.4 at 2 x 512; 30 M rows 23.5 ms
+// against 31.1 and 29.7); for k > 2 the rows' own gathers weigh more and the line is at 2048 rows a CU
+// (177 k rows, k = 4: 145 at 1 x 256, 167 at 1 x 1024; 735 k rows: 986 against 670).  Where they don't
+// fit, two lanes (1.9 M rows on 36 sites: 1698 at 2 x 512 against 1882; k = 4: 3509 at 2 x 256, 3856).
+static void lattice_shape(const dh_sector_set* S, int k, int* lpr, int* bs) {
+  *lpr = S->lanesPerRow;
+  *bs = S->blockSize;
+  if (!S->autoLaunch) return;
+  const int64_t perCU = S->totalDim / S->ctx->nbrCU;
+  auto set = [&](int l, int b) { *lpr = l, *bs = b; };
+  if (perCU < 128) return k <= 2 ? set(4, 256) : set(8, 256);
+  if (perCU < 512 && k <= 2) return set(2, 512);
+  if (lattice_lds(S, S->nbrSectors).factorsFit) return k > 2 && perCU < 2048 ? set(1, 256) : set(1, 1024);
+  k <= 2 ? set(2, 512) : set(2, 256);
 }
 
 template <int K>
 static int lattice_lpr(dh_sector_set* S, const double* x, double* y, int add, const unsigned char* active) {
-  switch (S->lanesPerRow) {
-    case 1: return lattice_launch<K, 1>(S, x, y, add, active);
-    case 2: return lattice_launch<K, 2>(S, x, y, add, active);
-    case 4: return lattice_launch<K, 4>(S, x, y, add, active);
-    default: return lattice_launch<K, 8>(S, x, y, add, active);
+  int lpr, bs;
+  lattice_shape(S, K, &lpr, &bs);
+  switch (lpr) {
+    case 1: return lattice_launch<K, 1>(S, bs, x, y, add, active);
+    case 2: return lattice_launch<K, 2>(S, bs, x, y, add, active);
+    case 4: return lattice_launch<K, 4>(S, bs, x, y, add, active);
+    default: return lattice_launch<K, 8>(S, bs, x, y, add, active);
   }
 }
 

@@ -243,6 +243,7 @@ extern "C" int dh_sector_set_launch(dh_sector_set* S, int lanesPerRow, int block
   if (blockSize < 64 || blockSize > 1024 || (blockSize % 64)) return dh_fail(S->ctx, DH_E_ARG, "block_size");
   S->lanesPerRow = lanesPerRow;
   S->blockSize = blockSize;
+  S->autoLaunch = false;
   return DH_OK;
 }
 

@@ -236,17 +236,15 @@ void LatticeSectorsBlockLanczos::SolveWave(const std::vector<int>& sectors, uint
   std::vector<int64_t> off(na + 1);
   dh_sector_set_offsets(S, off.data());
   const int64_t total = off.back();
-  // small sets: four lanes per row for enough wavefronts; large ones: the fastest shapes of N=10
-  // on 6 x 5 sites, 30 sectors, measured on MI355X: k <= 2 two lanes per row and 512-thread
-  // workgroups (39.9 ms at k = 1), k > 2 one lane per row and 256-thread workgroups (84.5 ms at
-  // k = 4, against 90.4 ms with two lanes and 512 threads)
+  // momentum sets pick their own launch per product; torus sets: four lanes per row for enough
+  // wavefronts when small
   if (Launch.lanesPerRow > 0)
     Arch->Check(dh_sector_set_launch(S, Launch.lanesPerRow, Launch.blockSize), "launch");
-  else if (total < 4ll * 256 * 256)
+  else if (TorusTranslations && total < 4ll * 256 * 256)
     Arch->Check(dh_sector_set_launch(S, 4, 256), "launch");
-  else if (k <= 2)
+  else if (TorusTranslations && k <= 2)
     Arch->Check(dh_sector_set_launch(S, 2, 512), "launch");
-  else
+  else if (TorusTranslations)
     Arch->Check(dh_sector_set_launch(S, 1, 256), "launch");
   std::vector<int64_t> dims(na);
   for (int i = 0; i < na; ++i) dims[i] = off[i + 1] - off[i];

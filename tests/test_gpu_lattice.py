@@ -137,3 +137,28 @@ def test_momentum_element_counts_match_oracle_rows(arch):
         expect = sum(len(O.fm_row_elements(ref, fac, r)[0]) for r in range(ref.dim))
         assert counts[i] == expect, (kx, ky, counts[i], expect)
     S.close()
+
+
+# 32 bits a word up to 32 orbitals, 64 above; the factors in LDS for 1024 threads where they fit
+# (30 orbitals, not 32); one row of momenta; no launch chosen (lpr 0)
+@pytest.mark.parametrize("n,nx,ny,lpr,block", [(3, 6, 5, 1, 1024), (3, 6, 5, 4, 1024), (4, 5, 3, 2, 1024),
+                                               (3, 8, 4, 1, 1024), (3, 1, 32, 1, 256), (3, 11, 3, 2, 256),
+                                               (2, 8, 5, 8, 64), (2, 1, 37, 1, 256), (4, 5, 4, 0, 0)])
+@pytest.mark.parametrize("k", [1, 2, 8])
+def test_momentum_rows_at_word_and_table_limits(arch, n, nx, ny, lpr, block, k):
+    sectors = [(0, 0), (nx - 1, 1), (nx // 2, ny - 1)]
+    S = MomentumSet(arch, n, nx, ny, sectors)
+    if lpr:
+        S.capi.gpu().dh_sector_set_launch(S.h, lpr, block)
+    u, _ = O.checkerboard_lower_band(nx, ny, T1, T2, TPP)
+    fac = O.LatticeFactors(nx, ny, u)
+    rng = np.random.default_rng(11)
+    X = rng.standard_normal((S.total, k)) + 1j * rng.standard_normal((S.total, k))
+    Y = S.hv(X, k)
+    for i, (kx, ky) in enumerate(sectors):
+        ref = O.MomentumFermions(n, nx, ny, kx, ky)
+        a, b = S.off[i], S.off[i + 1]
+        for v in range(k):
+            y_ref = O.fm_hv(ref, fac, X[a:b, v])
+            assert np.linalg.norm(Y[a:b, v] - y_ref) <= 1e-12 * np.linalg.norm(y_ref), (kx, ky, v)
+    S.close()
