@@ -206,8 +206,8 @@ struct dh_sector_set {
   double* d_phase = nullptr;   // per sector `modulo` (cos, sin) pairs
   int lutBits = 0, modulo = 1, stateShift = 0;
   int lanesPerRow = 1, blockSize = 256;
-  // momentum sets: pick lanes per row and workgroup size per product from k and the rows (until
-  // dh_sector_set_launch is called)
+  // sphere and momentum sets: pick lanes per row and workgroup size per product from k and the rows
+  // (until dh_sector_set_launch is called)
   bool autoLaunch = true;
   int rowMode = DH_INDEX_RANK;  // DH_INDEX_RANK, _FREE or _RANGE row routine
   // segmented BLAS launch shape: persistent axpy workgroups per CU, dots rows per tile (0: auto)

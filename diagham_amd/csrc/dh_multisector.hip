@@ -426,28 +426,35 @@ static SectorsArgs sectors_args(dh_sector_set* S, int nActive, int64_t totalTile
   return a;
 }
 
+// Dynamic LDS for `na` active sectors: the packed factors and the work list, with the 16-bit low rank
+// table when it exists and two workgroups' tables fit a CU's 160 KiB.
+static size_t sectors_lds(const dh_sector_set* S, int na, bool* loLds) {
+  const size_t base = ((size_t)S->nbrPackedFactors * 8 + (size_t)S->nbrPairSums * 4 + 7) / 8 * 8 + 8 * (2 * na + 1);
+  const size_t withLo = base + 2 * S->loSize;
+  *loLds = S->d_rankLo16 && withLo <= 79 * 1024;
+  return *loLds ? withLo : base;
+}
+
 template <int K, int LPR>
-static int sectors_hv_launch(dh_sector_set* S, const double* x, double* y, int add, const unsigned char* active) {
+static int sectors_hv_launch(dh_sector_set* S, int blockSize, const double* x, double* y, int add,
+                             const unsigned char* active) {
   dh_context* c = S->ctx;
-  int64_t rowsPerTile = S->blockSize / LPR;
+  int64_t rowsPerTile = blockSize / LPR;
   int na;
   int64_t tiles;
   int rc = dh_sectors_upload_work(S, active, rowsPerTile, &na, &tiles);
   if (rc) return rc;
   if (tiles == 0) return DH_OK;
-  size_t base = ((size_t)S->nbrPackedFactors * 8 + (size_t)S->nbrPairSums * 4 + 7) / 8 * 8 + 8 * (2 * na + 1);
-  // the 16-bit low table in LDS when it exists and two workgroups' tables fit a CU's 160 KiB
-  size_t withLo = base + 2 * S->loSize;
-  bool loLds = S->d_rankLo16 && withLo <= 79 * 1024;
-  size_t lds = loLds ? withLo : base;
+  bool loLds;
+  const size_t lds = sectors_lds(S, na, &loLds);
   if (lds > 160 * 1024) return dh_fail(c, DH_E_RANGE, "staged tables exceed LDS");
   SectorsArgs a = sectors_args(S, na, tiles);
   auto launch = [&](auto kern) -> int {
     if (lds > 64 * 1024)
       DH_HIP(c, hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    const int perCU = dh_blocks_per_cu(c, kern, S->blockSize, lds);
+    const int perCU = dh_blocks_per_cu(c, kern, blockSize, lds);
     int64_t grid = std::max<int64_t>(1, std::min<int64_t>(tiles, (int64_t)c->nbrCU * perCU));
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(S->blockSize), lds, c->stream, a, x, y, add);
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(blockSize), lds, c->stream, a, x, y, add);
     DH_HIP(c, hipGetLastError());
     return DH_OK;
   };
@@ -470,13 +477,39 @@ static int sectors_hv_launch(dh_sector_set* S, const double* x, double* y, int a
   return loLds ? pick(std::true_type{}, std::false_type{}) : pick(std::false_type{}, std::false_type{});
 }
 
+// Lanes per row and workgroup size by rows per CU and k, times in us on MI355X (the set's default was
+// 1 x 256).  Few rows: lanes for wavefronts (26 k rows: 20.1 with 2 x 256, 22.9; 4173 rows, k = 4: 16.7
+// with 8 x 256, 33.0).  To 2048 rows a CU small workgroups spread best (164 k rows: 39.7 with 1 x 256,
+// 45 with 1 x 512 and 1 x 1024; k = 4: 80 with 2 x 256, 96 with 1 x 256).  Above, the tables in LDS bound
+// the wavefronts of a CU: 512 threads when three workgroups fit it, else 1024 (1.0 M rows: 205 and 215,
+// 248 at 256; 17.6 M rows with 29 orbitals, two workgroups: 5.4 ms at 1024, 8.4 at 512, 14.0 at 256;
+// k = 4, 6.7 M rows, three: 4.7 ms at 512, 6.5 at 1024, 8.1 at 256).  k = 8 and 16: two lanes, 512 (1.0 M
+// rows 943 against 1012 and 2178 against 2934), except k = 8 with many rows (6.7 M: 8.6 ms with 1 x 1024,
+// 9.5 with 2 x 512).
+static void sectors_shape(const dh_sector_set* S, int k, int* lpr, int* bs) {
+  *lpr = S->lanesPerRow;
+  *bs = S->blockSize;
+  if (!S->autoLaunch) return;
+  const int64_t perCU = S->totalDim / S->ctx->nbrCU;
+  auto set = [&](int l, int b) { *lpr = l, *bs = b; };
+  if (perCU < 128) return k <= 2 ? set(2, 256) : set(8, 256);
+  if (perCU < 2048) return k <= 2 ? set(1, 256) : set(2, 256);
+  if (k > 8 || (k == 8 && perCU < 8192)) return set(2, 512);
+  bool lo;
+  const bool three = 3 * sectors_lds(S, S->nbrSectors, &lo) <= 160 * 1024;
+  if (k == 8 || !three || (k <= 2 && perCU >= 8192)) return set(1, 1024);
+  set(1, 512);
+}
+
 template <int K>
 static int sectors_hv_lpr(dh_sector_set* S, const double* x, double* y, int add, const unsigned char* active) {
-  switch (S->lanesPerRow) {
-    case 1: return sectors_hv_launch<K, 1>(S, x, y, add, active);
-    case 2: return sectors_hv_launch<K, 2>(S, x, y, add, active);
-    case 4: return sectors_hv_launch<K, 4>(S, x, y, add, active);
-    default: return sectors_hv_launch<K, 8>(S, x, y, add, active);
+  int lpr, bs;
+  sectors_shape(S, K, &lpr, &bs);
+  switch (lpr) {
+    case 1: return sectors_hv_launch<K, 1>(S, bs, x, y, add, active);
+    case 2: return sectors_hv_launch<K, 2>(S, bs, x, y, add, active);
+    case 4: return sectors_hv_launch<K, 4>(S, bs, x, y, add, active);
+    default: return sectors_hv_launch<K, 8>(S, bs, x, y, add, active);
   }
 }
 

@@ -164,19 +164,11 @@ void MultiSectorBlockLanczos::SolveWave(const std::vector<int>& sectors, uint64_
   std::vector<int64_t> off(na + 1);
   dh_sector_set_offsets(S, off.data());
   const int64_t total = off.back();
-  // small sets: more lanes per row for enough wavefronts; large ones: the fastest shapes of the
-  // all-sector product of N=12 2S=33 measured on MI355X (k >= 4: two lanes per row, 1024-thread
-  // workgroups; k < 4: one lane per row, 1024-thread workgroups, 236 ms against 416 ms at 256
-  // threads: the workgroup's tables, with the 16-bit low rank table, take ~61 KiB of LDS)
+  // without a chosen shape the set picks its own per product
   if (Launch.lanesPerRow > 0) {
     Arch->Check(dh_sector_set_launch(S, Launch.lanesPerRow, Launch.blockSize), "launch");
     Arch->Check(dh_sector_set_row_mode(S, Launch.rowMode), "row mode");
-  } else if (total < 4ll * 256 * 256)
-    Arch->Check(dh_sector_set_launch(S, 4, 512), "launch");
-  else if (BlockSize >= 4)
-    Arch->Check(dh_sector_set_launch(S, 2, 1024), "launch");
-  else
-    Arch->Check(dh_sector_set_launch(S, 1, 1024), "launch");
+  }
   std::vector<int64_t> dims(na);
   for (int i = 0; i < na; ++i) dims[i] = off[i + 1] - off[i];
   std::vector<int> blockCap;

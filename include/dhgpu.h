@@ -150,12 +150,8 @@ int64_t dh_hamiltonian_dimension(const dh_hamiltonian* ham);
 /* Launch shape of the H.v kernels.  lanes_per_row in {1,2,4,8} (64/lanes_per_row destination
  * rows per wavefront; spin chains: 1); block_size a multiple of 64 up to 1024; index_mode
  * DH_INDEX_*; lds_tables != 0 stages the index tables in LDS when they fit.  Until it is called, a
- * sphere Hamiltonian picks its shape per product: on spaces of at least 256 rows per CU the
- * fastest shapes measured on N=12 2S=33 Lz=0 (with the 16-bit low rank table in LDS: one lane per
- * row, 1024-thread workgroups for k = 1, two lanes per row for k = 2, 512 threads for k > 2; with the
- * rank tables in global memory:
- * two lanes per row, 256 threads for k <= 2 and 1024 above); on smaller spaces four lanes per row,
- * 512 threads. */
+ * sphere Hamiltonian picks its shape per product from k and its rows per CU: more lanes per row in
+ * small workgroups on small spaces, 1024-thread workgroups on large ones. */
 int dh_hamiltonian_set_launch(dh_hamiltonian* ham, int lanes_per_row, int block_size, int index_mode, int lds_tables);
 
 /* ---------------------------------------------------------------- products
@@ -213,6 +209,8 @@ int dh_sector_set_get_states(dh_sector_set* set, uint64_t* states);
 /* factors in the dh_sphere_hamiltonian_create layout (shared by every sector) and the shift */
 int dh_sector_set_factors(dh_sector_set* set, const double* factors, const int* pair_offset, int nbr_factors,
                           double shift);
+/* Launch shape of the set's products.  Until it is called, sphere and momentum sets pick their shape
+ * per product from k and their rows per CU. */
 int dh_sector_set_launch(dh_sector_set* set, int lanes_per_row, int block_size);
 /* Row routine of the products of a sphere or momentum set: DH_INDEX_RANK_RANGE (every created pair
  * of the range or list, skipping occupied ones), DH_INDEX_RANK_FREE (only the free created pairs,
