@@ -526,24 +526,24 @@ static int sphere_dispatch_lpr(dh_hamiltonian* h, const double* x, double* y, in
   if (h->autoLaunch) {
     // the fastest shapes measured on MI355X by rows per CU and k, times in us.  Few rows: lanes for
     // wavefronts, in small workgroups (338 rows: 9.1 with 2 x 256, 10.2 with 4 x 512; 45 k rows: 26.2 with
-    // 2 x 512, 36.8 with 4 x 512; 71 k rows: 38.0 with 1 x 512, 53 with 1 x 1024; k = 8, 8512 rows: 23.3
-    // with 8 x 256, 31.8 with 4 x 512).  Many rows: with the 16-bit low table in LDS a workgroup holds
-    // about 60 KiB, two per CU, so 1024 threads (1.4 M rows: 603, 645 at 512; k = 4: 1436, 2068 at 512).
-    // k = 8 and 16 wait for their 64- and 128-byte gathers: two lanes (1.4 M rows: 2838 against 2898 and
-    // 6450 against 7300), and k = 8 one lane and 512 threads past 8192 rows a CU (7.8 M rows: 20.7 ms
-    // against 22.5).  With both tables in global memory: two lanes per row, 256 threads for k <= 2, 1024
-    // above.
+    // 2 x 512, 36.8 with 4 x 512; 71 k rows: 37.9 with 1 x 512, 53 with 1 x 1024 and 2 x 256, k = 4 81 with
+    // 2 x 1024, 110 and more with one lane; k = 8, 8512 rows: 23.3 with 8 x 256, 31.8 with 4 x 512).  Many
+    // rows: with the 16-bit low table in LDS a workgroup holds about 60 KiB, two per CU, so 1024 threads
+    // (1.4 M rows: 603, 645 at 512; k = 4: 1436, 2068 at 512).  k = 8 and 16 wait for their 64- and
+    // 128-byte gathers: two lanes (1.4 M rows: 2838 against 2898 and 6450 against 7300), and k = 8 one lane
+    // and 512 threads past 8192 rows a CU (7.8 M rows: 20.7 ms against 22.5).  With both tables in global
+    // memory: two lanes per row, 256 threads for k <= 2, 1024 above.
     const int64_t perCU = h->basis->dim / h->ctx->nbrCU;
     auto set = [&](int l, int b) { lpr = l, bs = b; };
     if (perCU < 64)
       K <= 2 ? set(2, 256) : set(8, 256);
     else if (perCU < 256)
       K <= 2 ? set(2, 512) : set(4, 1024);
-    else if (sphere_rank_tables(h) != MODE_RANK_LO16)
+    else if (sphere_rank_tables(h) == MODE_RANK_GLOBAL)
       set(2, K <= 2 ? 256 : 1024);
     else if (K == 1)
       set(1, perCU < 512 ? 512 : 1024);
-    else if (K == 4)
+    else if (K == 4 && perCU >= 512)
       set(1, 1024);
     else if (K == 8 && perCU >= 8192)
       set(1, 512);
