@@ -293,6 +293,10 @@ extern "C" int dh_spin_chain_create(dh_context* c, dh_basis** out, int L, int sz
   }
   hipLaunchKernelGGL(spin_lut_kernel, dim3((unsigned)(((1 << b->lutBits) + 1 + 255) / 256)), dim3(256), 0,
                      c->stream, b->d_words, dim, L, b->lutShift, b->lutBits, b->d_lut);
+  if (L >= 20 && (rc = dh_spin_tile_tables(b))) {
+    dh_basis_destroy(b);
+    return rc;
+  }
   hipError_t e = hipStreamSynchronize(c->stream);
   if (e != hipSuccess) {
     dh_basis_destroy(b);
@@ -309,6 +313,7 @@ extern "C" int dh_basis_destroy(dh_basis* b) {
   hipStreamSynchronize(c->stream);
   if (b->d_states) hipFree(b->d_states);
   if (b->d_words) hipFree(b->d_words);
+  if (b->d_spinTile) hipFree(b->d_spinTile);
   if (b->d_lut) hipFree(b->d_lut);
   if (b->d_rankLo) hipFree(b->d_rankLo);
   if (b->d_rankHi) hipFree(b->d_rankHi);

@@ -108,6 +108,7 @@ struct dh_basis {
   uint16_t* d_rankLo16 = nullptr;
   // binomial table C[n][k], n,k <= 32 (spin rank)
   uint32_t* d_binom = nullptr;
+  uint32_t* d_spinTile = nullptr;  // pattern tables of the tiled spin product (dh_spin_tile_tables)
 };
 
 enum dh_ham_kind { DH_HAM_SPHERE = 1, DH_HAM_SPIN = 2, DH_HAM_SPHERE_NBODY = 3 };
@@ -221,6 +222,12 @@ struct dh_sector_set {
 };
 
 // work descriptor of the active sectors (dh_multisector.hip)
+// tiled spin-1/2 product (dh_spin_tile.hip): its tables, whether it takes blocks of k, the product
+int dh_spin_tile_tables(dh_basis* b);
+bool dh_spin_tiles(const dh_hamiltonian* h, int k);
+int dh_spin_tile_hv(dh_hamiltonian* h, bool uniform, const double* x, double* y, int k, int add, int64_t first,
+                    int64_t count);
+
 int dh_sectors_upload_work(dh_sector_set* S, const unsigned char* active, int64_t rowsPerTile, int* nActive,
                            int64_t* totalTiles);
 // complex product over a momentum set and its matrix elements per sector (dh_lattice.hip)

@@ -99,3 +99,38 @@ def test_lanczos_l24_reference_eigenvalues(arch, golden):
     assert r["converged"]
     np.testing.assert_allclose(r["eigenvalues"], ref, rtol=0, atol=1e-10)
     p.close()
+
+
+# the tiled product: every number of last sites, tiles of one row (Sz = 0 has them), partly filled ones
+@pytest.mark.parametrize("L,sz,periodic,k,uniform", [(21, 1, True, 1, True), (22, -2, False, 1, False),
+                                                     (26, 0, True, 1, False), (22, 0, True, 2, True),
+                                                     (22, 2, False, 2, False), (21, -1, True, 4, False),
+                                                     (20, 0, True, 8, False), (20, 2, False, 8, True),
+                                                     (20, 0, True, 16, True), (20, 0, False, 16, False)])
+def test_hv_by_tiles(arch, L, sz, periodic, k, uniform):
+    from diagham_amd import capi
+    rng = np.random.default_rng(L + k)
+    J = np.full(L, 0.7) if uniform else rng.uniform(0.5, 1.5, L)
+    Jz = np.full(L, 1.3) if uniform else rng.uniform(0.5, 1.5, L)
+    p = capi.Problem.spin_chain(arch, L, sz, J, Jz, periodic)
+    ref = O.SpinChain(L, sz)
+    X = np.stack([O.splitmix(400 + v, p.dim) for v in range(k)], axis=1)
+    Y = p.hv(X.reshape(-1), k).reshape(p.dim, k)
+    for v in {0, k - 1}:
+        x = np.ascontiguousarray(X[:, v])
+        y_ref = np.zeros_like(x)
+        O.lib().or_spin_hv(ref.h, O.dptr(J), O.dptr(Jz), int(periodic), O.dptr(x), O.dptr(y_ref))
+        err = np.linalg.norm(Y[:, v] - y_ref) / np.linalg.norm(y_ref)
+        assert err < 1e-12, (L, sz, periodic, k, v, err)
+    # row ranges, added to what is there: the same values, and no other row touched
+    cuts = [0, 1, 2, p.dim // 3, p.dim // 3 + 1, p.dim // 2 + 5, p.dim - 1, p.dim]
+    base = O.splitmix(500, p.dim * k)
+    dx = capi.DeviceBuffer.from_host(arch, X.reshape(-1))
+    for a, b in zip(cuts, cuts[1:]):
+        dy = capi.DeviceBuffer.from_host(arch, base)
+        p.hv_device(dx.ptr, dy.ptr, k, add=True, first=a, count=b - a)
+        out = dy.download().reshape(p.dim, k)
+        expect = base.reshape(p.dim, k).copy()
+        expect[a:b] += Y[a:b]
+        assert np.array_equal(out, expect), (a, b)
+    p.close()
