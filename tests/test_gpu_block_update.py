@@ -101,3 +101,21 @@ def test_sectors_block_update_matches_numpy(arch, k):
     dV.free()
     dW.free()
     S.close()
+
+
+# few rows: dot products in one kernel up to 16384 rows, the update split over wavefronts up to 131072 rows
+# and 448 vectors (at most 8 take a kernel of their own); odd row numbers read no pairs
+@pytest.mark.parametrize("dim,nb", [(d, n) for d in (1, 63, 129, 8513, 16384, 16386, 131071, 131073)
+                                    for n in (1, 9, 64, 65, 450) if d < 20000 or n <= 65])
+def test_dots_and_axpy_of_few_rows(arch, dim, nb):
+    from diagham_amd import capi
+    rng = np.random.default_rng(dim + nb)
+    V, W, C = rng.standard_normal((nb, dim)), rng.standard_normal(dim), rng.standard_normal(nb)
+    dV, dW = capi.DeviceBuffer.from_host(arch, V.reshape(-1)), capi.DeviceBuffer.from_host(arch, W)
+    out = np.zeros(nb)
+    assert capi.gpu().dh_block_dots(arch.ctx, dV.ptr, nb, dW.ptr, dim, 1, capi.dptr(out)) == 0
+    # rounding of a sum of dim products in any order: at most dim eps times the sum of their magnitudes
+    assert (np.abs(out - V @ W) <= 1e-15 * dim * (np.abs(V) @ np.abs(W)) + 1e-300).all()
+    assert capi.gpu().dh_block_axpy(arch.ctx, dV.ptr, nb, dW.ptr, dim, 1, capi.dptr(C)) == 0
+    mag = np.abs(W) + np.abs(C) @ np.abs(V)
+    assert (np.abs(dW.download() - (W + C @ V)) <= 1e-15 * (nb + 1) * mag).all()
