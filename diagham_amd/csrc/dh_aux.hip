@@ -352,104 +352,129 @@ extern "C" int dh_hamiltonian_row_elements(dh_hamiltonian* h, int64_t row, int64
 //   A_c(v)[t] = sum_{pairs p free in t, sum(p) = sum(s) - sum(t)} u_c[p] (-1)^(popc(t >> p_lo) + popc(t >> p_hi)) v[t | p]
 // (the annihilation sign of a pair is its creation sign plus one, and the two cancel).  Each (row,
 // annihilated pair, created pair) term of the product becomes one (t, pair) term here, so a
-// bilinear costs C(N, 2) gathers per row instead of one per matrix element.  One lane per t, the
-// t unranked from its index in the combinatorial number system over all (N-2)-subsets of the
-// orbitals; the index loads, then the gathers, of four pairs are in flight together.  SAME: psi and
-// phi are the same vector (an expectation value), one sum per channel.  Channels [c0, c0 + NC).
-template <int NC, bool SAME>
-__global__ void __launch_bounds__(256) sphere_adjoint_kernel(int nbrOrbitals, int holes, int64_t nbrSubsets,
-                                                             int orbitalSum, const int64_t* __restrict__ binom,
-                                                             int nbrChannels, int c0, const double* __restrict__ cg,
-                                                             int nbrPairs, const uint32_t* __restrict__ lo,
-                                                             const uint32_t* __restrict__ hi, int rankBits,
-                                                             int64_t dim, const double* __restrict__ psi,
-                                                             const double* __restrict__ phi,
-                                                             double* __restrict__ partial) {
+// bilinear costs C(N, 2) gathers per row instead of one per matrix element.  A lane takes `run`
+// (N-2)-subsets of the orbitals in a row: the first one unranked from its index in the combinatorial
+// number system, the others by the next word with as many bits.  The index loads, then the gathers, of
+// four pairs are in flight together.  SAME: psi and phi are the same vector (an expectation value), one sum
+// per channel.  Channels [c0, c0 + NC), U: words of 32 bits when the orbitals fit.
+//
+// The channel table is channel-major: a lane reads NC coefficients of its own pair, and with pairs as rows of
+// 128 bytes the lanes met in a few LDS banks, 81 % of the LDS cycles and the bound (N=10 2S=27, 14 channels:
+// 274 us; 167 and 205 with rows padded to 18 and 17 doubles, 125 channel-major).  With words of 32 bits, masks over
+// positions, runs of up to 8 subsets and 512 threads: 86 (256 threads 95, 1024 96; runs of one 107).
+__device__ __forceinline__ int dh_bit_sum(uint32_t t) {  // sum of the positions of the set bits
+  return __popc(t & 0xaaaaaaaau) + 2 * __popc(t & 0xccccccccu) + 4 * __popc(t & 0xf0f0f0f0u) +
+         8 * __popc(t & 0xff00ff00u) + 16 * __popc(t & 0xffff0000u);
+}
+__device__ __forceinline__ int dh_bit_sum(uint64_t t) {
+  return dh_bit_sum((uint32_t)t) + dh_bit_sum((uint32_t)(t >> 32)) + 32 * __popc((uint32_t)(t >> 32));
+}
+
+constexpr int kAdjointThreads = 512;
+template <int NC, bool SAME, typename U>
+__global__ void __launch_bounds__(kAdjointThreads) sphere_adjoint_kernel(int nbrOrbitals, int holes, int64_t nbrSubsets, int run,
+                                                            int orbitalSum, const int64_t* __restrict__ binom,
+                                                            int nbrChannels, int c0, const double* __restrict__ cg,
+                                                            int nbrPairs, const uint32_t* __restrict__ lo,
+                                                            const uint32_t* __restrict__ hi, int rankBits,
+                                                            uint32_t last, const double* __restrict__ psi,
+                                                            const double* __restrict__ phi,
+                                                            double* __restrict__ partial) {
+  constexpr int BD = kAdjointThreads;
   extern __shared__ double smem[];
-  double* sU = smem;                                                 // [nbrPairs][NC]
+  double* sU = smem;                                                 // [NC][nbrPairs]
   int64_t* sB = reinterpret_cast<int64_t*>(smem + nbrPairs * NC);    // [nbrOrbitals + 1][holes + 1]
-  __shared__ double red[256 / 64][NC];
+  __shared__ double red[BD / 64][NC];
   const int nc = min(NC, nbrChannels - c0);
-  for (int i = threadIdx.x; i < nbrPairs * NC; i += blockDim.x) {
+  for (int i = threadIdx.x; i < nbrPairs * NC; i += BD) {
     const int p = i / NC, c = i - p * NC;
-    sU[i] = c < nc ? cg[(int64_t)p * nbrChannels + c0 + c] : 0.0;
+    sU[c * nbrPairs + p] = c < nc ? cg[(int64_t)p * nbrChannels + c0 + c] : 0.0;
   }
-  for (int i = threadIdx.x; i < (nbrOrbitals + 1) * (holes + 1); i += blockDim.x) sB[i] = binom[i];
+  for (int i = threadIdx.x; i < (nbrOrbitals + 1) * (holes + 1); i += BD) sB[i] = binom[i];
   __syncthreads();
   double g[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) g[c] = 0.0;
   const int maxSum = 2 * nbrOrbitals - 3;
-  for (int64_t it = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; it < nbrSubsets;
-       it += (int64_t)gridDim.x * blockDim.x) {
+  const U loMask = (U(1) << rankBits) - U(1);
+  for (int64_t it = ((int64_t)blockIdx.x * BD + threadIdx.x) * run; it < nbrSubsets; it += (int64_t)gridDim.x * BD * run) {
     // the it-th (N-2)-subset: it = sum_k C(c_k, k) over its orbitals c_1 < ... < c_m
-    uint64_t t = 0;
+    U t = 0;
     int64_t r = it;
-    int m = holes, sumT = 0;
+    int m = holes;
     for (int j = nbrOrbitals - 1; j >= 0 && m > 0; --j) {
       const int64_t b = sB[j * (holes + 1) + m];
       if (r >= b) {
-        t |= 1ull << j;
-        sumT += j;
+        t |= U(1) << j;
         r -= b;
         --m;
       }
     }
-    const int S = orbitalSum - sumT;  // the pair sum that completes t to the sector
-    if (S < 1 || S > maxSum) continue;
-    uint64_t pm = dh_free_pairs(t, nbrOrbitals, S, (S >> 1) + 1, min(S, nbrOrbitals - 1));
-    if (!pm) continue;
-    double a[NC], bsum[SAME ? 1 : NC];
+    const int n = (int)min((int64_t)run, nbrSubsets - it);
+    for (int step = 0; step < n; ++step) {
+      if (step > 0) {  // the next larger word with as many bits (there is one: at least one bit is set)
+        const U low = t & (U(0) - t), up = t + low;
+        t = up | (((up ^ t) >> 2) >> dh_ctz(low));
+      }
+      const int S = orbitalSum - dh_bit_sum(t);  // the pair sum that completes t to the sector
+      if (S < 1 || S > maxSum) continue;
+      const dh_row_masks<U> masks(t, nbrOrbitals);
+      const int m3lo = (S >> 1) + 1, m4hi = (S - 1) >> 1;
+      uint32_t pm = masks.free(m3lo, m4hi);
+      if (!pm) continue;
+      const uint32_t sg = masks.sign(m3lo, m4hi);
+      double a[NC], bsum[SAME ? 1 : NC];
 #pragma unroll
-    for (int c = 0; c < NC; ++c) a[c] = 0.0;
-    if constexpr (!SAME) {
+      for (int c = 0; c < NC; ++c) a[c] = 0.0;
+      if constexpr (!SAME) {
 #pragma unroll
-      for (int c = 0; c < NC; ++c) bsum[c] = 0.0;
-    }
-    while (pm) {
-      int64_t idx[4];
-      int pb[4];
-      bool neg[4];
+        for (int c = 0; c < NC; ++c) bsum[c] = 0.0;
+      }
+      while (pm) {
+        uint32_t idx[4];
+        int pos[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        idx[q] = 0;  // a slot past the last pair reads row 0 with no weight
-        pb[q] = -1;
-        neg[q] = false;
-        if (pm) {
-          const int m3 = __builtin_ctzll(pm);
-          pm &= pm - 1;
-          const int m4 = S - m3;
-          idx[q] = dh_find_rank(t | (1ull << m3) | (1ull << m4), lo, hi, rankBits, dim);
-          pb[q] = (m3 * (m3 - 1)) / 2 + m4;
-          neg[q] = (__popcll(t >> m4) + __popcll(t >> m3)) & 1;
+        for (int q = 0; q < 4; ++q) {
+          idx[q] = 0;  // a slot past the last pair reads row 0 with no weight
+          pos[q] = -1;
+          if (pm) {
+            const int i = __builtin_ctz(pm);
+            pm &= pm - 1;
+            const U w = t | (U(1) << (m3lo + i)) | (U(1) << (m4hi - i));
+            // clamped so that a target outside the sector can never address outside the vectors
+            idx[q] = min(dh_word(hi, (uint32_t)(w >> rankBits)) - dh_word(lo, (uint32_t)(w & loMask)), last);
+            pos[q] = i;
+          }
+        }
+        double x[4], z[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          x[q] = psi[idx[q]];
+          if constexpr (!SAME) z[q] = phi[idx[q]];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if (pos[q] < 0) continue;
+          const int m3 = m3lo + pos[q];
+          const double* u = sU + (__mul24(m3, m3 - 1) / 2 + m4hi - pos[q]);
+          const uint32_t neg = sg << (31 - pos[q]);
+          const double xs = dh_negate_by(x[q], neg);
+#pragma unroll
+          for (int c = 0; c < NC; ++c) a[c] += u[c * nbrPairs] * xs;
+          if constexpr (!SAME) {
+            const double zs = dh_negate_by(z[q], neg);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) bsum[c] += u[c * nbrPairs] * zs;
+          }
         }
       }
-      double x[4], z[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        x[q] = psi[idx[q]];
-        if constexpr (!SAME) z[q] = phi[idx[q]];
+      for (int c = 0; c < NC; ++c) {
+        if constexpr (SAME)
+          g[c] += a[c] * a[c];
+        else
+          g[c] += a[c] * bsum[c];
       }
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        if (pb[q] < 0) continue;
-        const double* u = sU + (int64_t)pb[q] * NC;
-        const double xs = neg[q] ? -x[q] : x[q];
-#pragma unroll
-        for (int c = 0; c < NC; ++c) a[c] += u[c] * xs;
-        if constexpr (!SAME) {
-          const double zs = neg[q] ? -z[q] : z[q];
-#pragma unroll
-          for (int c = 0; c < NC; ++c) bsum[c] += u[c] * zs;
-        }
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      if constexpr (SAME)
-        g[c] += a[c] * a[c];
-      else
-        g[c] += a[c] * bsum[c];
     }
   }
   const int wl = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -512,30 +537,41 @@ static int64_t adjoint_binomials(dh_hamiltonian* h, int holes, int* rc) {
   return total;
 }
 
-template <int NC, bool SAME>
+template <int NC, bool SAME, typename U>
 static int adjoint_pass(dh_hamiltonian* h, int holes, int64_t subsets, int c0, const double* psi, const double* phi,
                         double* g) {
   dh_context* c = h->ctx;
   dh_basis* b = h->basis;
   size_t lds = sizeof(double) * h->nbrPairs * NC + sizeof(int64_t) * (b->nbrOrbitals + 1) * (holes + 1);
   if (lds > 150 * 1024) return dh_fail(c, DH_E_RANGE, "channel table exceeds LDS");
-  auto kern = sphere_adjoint_kernel<NC, SAME>;
+  constexpr int BD = kAdjointThreads;
+  auto kern = sphere_adjoint_kernel<NC, SAME, U>;
   if (lds > 64 * 1024) DH_HIP(c, hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  const int perCU = dh_blocks_per_cu(c, kern, 256, lds);
-  int nb = (int)std::max<int64_t>(1, std::min<int64_t>((subsets + 255) / 256, (int64_t)c->nbrCU * std::max(perCU, 1)));
+  const int perCU = dh_blocks_per_cu(c, kern, BD, lds);
+  // runs of up to 8 subsets, while there are enough of them for every lane
+  const int64_t lanes = (int64_t)c->nbrCU * perCU * BD;
+  const int run = (int)std::max<int64_t>(1, std::min<int64_t>(8, subsets / lanes));
+  const int64_t want = (subsets + (int64_t)BD * run - 1) / ((int64_t)BD * run);
+  int nb = (int)std::max<int64_t>(1, std::min<int64_t>(want, (int64_t)c->nbrCU * perCU));
   double* scratch;
-  int rc = dh_scratch(c, sizeof(double) * ((size_t)nb * NC + NC), &scratch);
-  if (rc) return rc;
-  hipLaunchKernelGGL(kern, dim3(nb), dim3(256), lds, c->stream, b->nbrOrbitals, holes, subsets, b->orbitalSum,
+  double* out;  // pinned: the sums are written where the host reads them
+  int rc = dh_scratch(c, sizeof(double) * (size_t)nb * NC, &scratch);
+  if (rc || (rc = dh_pinned(c, sizeof(double) * NC, &out))) return rc;
+  hipLaunchKernelGGL(kern, dim3(nb), dim3(BD), lds, c->stream, b->nbrOrbitals, holes, subsets, run, b->orbitalSum,
                      (const int64_t*)h->d_adjBinom, h->nbrChannels, c0, h->d_cg, h->nbrPairs, b->d_rankLo,
-                     b->d_rankHi, b->rankBits, b->dim, psi, phi, scratch);
-  hipLaunchKernelGGL(reduce_partials_kernel, dim3(NC), dim3(256), 0, c->stream, scratch, nb, NC, scratch + (size_t)nb * NC);
+                     b->d_rankHi, b->rankBits, (uint32_t)b->dim - 1u, psi, phi, scratch);
+  hipLaunchKernelGGL(reduce_partials_kernel, dim3(NC), dim3(256), 0, c->stream, scratch, nb, NC, out);
   DH_HIP(c, hipGetLastError());
-  double out[NC];
-  DH_HIP(c, hipMemcpyAsync(out, scratch + (size_t)nb * NC, sizeof(double) * NC, hipMemcpyDeviceToHost, c->stream));
   DH_HIP(c, hipStreamSynchronize(c->stream));
   for (int i = 0; i < NC && c0 + i < h->nbrChannels; ++i) g[c0 + i] = out[i];
   return DH_OK;
+}
+
+template <int NC, bool SAME>
+static int adjoint_words(dh_hamiltonian* h, int holes, int64_t subsets, int c0, const double* psi, const double* phi,
+                         double* g) {
+  if (h->basis->nbrOrbitals <= 32) return adjoint_pass<NC, SAME, uint32_t>(h, holes, subsets, c0, psi, phi, g);
+  return adjoint_pass<NC, SAME, uint64_t>(h, holes, subsets, c0, psi, phi, g);
 }
 
 extern "C" int dh_sphere_adjoint(dh_hamiltonian* h, const double* psi, const double* phi, double* g, double* hpsi) {
@@ -562,11 +598,11 @@ extern "C" int dh_sphere_adjoint(dh_hamiltonian* h, const double* psi, const dou
   for (int c0 = 0; c0 < h->nbrChannels; c0 += 16) {
     const int left = h->nbrChannels - c0;
     if (left <= 8)
-      rc = same ? adjoint_pass<8, true>(h, holes, subsets, c0, psi, phi, g)
-                : adjoint_pass<8, false>(h, holes, subsets, c0, psi, phi, g);
+      rc = same ? adjoint_words<8, true>(h, holes, subsets, c0, psi, phi, g)
+                : adjoint_words<8, false>(h, holes, subsets, c0, psi, phi, g);
     else
-      rc = same ? adjoint_pass<16, true>(h, holes, subsets, c0, psi, phi, g)
-                : adjoint_pass<16, false>(h, holes, subsets, c0, psi, phi, g);
+      rc = same ? adjoint_words<16, true>(h, holes, subsets, c0, psi, phi, g)
+                : adjoint_words<16, false>(h, holes, subsets, c0, psi, phi, g);
     if (rc) return rc;
   }
   return DH_OK;

@@ -220,19 +220,3 @@ __device__ __forceinline__ void dh_sphere_row_x4(U s, int nbrOrbitals, const dou
   }
   if (lane == 0) dh_gather_fma<K>(acc, xbase, self, diag);
 }
-
-// Created pairs (m3 > m4, m3 + m4 = sum, both orbitals free in t) as a mask of their m3 bits:
-// bit m of f & (f mirrored about sum / 2) says that m and sum - m are both free.  The mirror of f
-// is its bit reversal within the nbrOrbitals orbitals, shifted so that bit sum - m lands on bit m.
-template <typename U>
-__device__ __forceinline__ U dh_free_pairs(U t, int nbrOrbitals, int sum, int m3lo, int m3hi) {
-  constexpr int W = 8 * sizeof(U);
-  const U full = nbrOrbitals >= W ? ~U(0) : ((U(1) << nbrOrbitals) - U(1));
-  const U f = ~t & full;
-  const U g = dh_bitrev(f) >> (W - nbrOrbitals);  // bit j of g = bit nbrOrbitals - 1 - j of f
-  const int d = nbrOrbitals - 1 - sum;             // bit m of the mirror = bit m + d of g
-  const U mirror = d >= 0 ? (g >> d) : (g << (-d));
-  const U hiMask = m3hi >= W - 1 ? ~U(0) : ((U(1) << (m3hi + 1)) - U(1));
-  const U loMask = (U(1) << m3lo) - U(1);
-  return f & mirror & hiMask & ~loMask;
-}

@@ -213,3 +213,27 @@ def test_l0_gap_gradients_match_finite_differences(arch):
         assert abs(a - b) <= 1e-6 * abs(b) + 4 * noise, ("dGap", m, a, b)
     for q in (shifted, L2, p):
         q.close()
+
+
+@pytest.mark.parametrize("n,total_lz,lz", [(10, 0, 25), (7, 1, 39), (2, 0, 3)])
+def test_bilinears_by_runs_match_products(arch, n, total_lz, lz):
+    """Several (N-2)-subsets per lane (32- and 64-bit words, one and two channel groups), and the one
+    empty subset: <psi|H_m|phi> against the product of H_m alone."""
+    from diagham_amd import capi
+    rng = np.random.default_rng(n)
+    p = capi.Problem.sphere(arch, n, total_lz, lz, rng.uniform(0.1, 1.0, lz + 1))
+    psi, phi = rng.standard_normal(p.dim), rng.standard_normal(p.dim)
+    dpsi, dphi = capi.DeviceBuffer.from_host(arch, psi), capi.DeviceBuffer.from_host(arch, phi)
+    g = p.adjoint_device(dpsi.ptr, dphi.ptr)
+    gs = p.adjoint_device(dpsi.ptr, dpsi.ptr)
+    channels = list(p.channels())
+    p.close()
+    for c in {0, len(channels) // 2, len(channels) - 1}:
+        V = np.zeros(lz + 1)
+        V[channels[c]] = 1.0
+        q = capi.Problem.sphere(arch, n, total_lz, lz, V)
+        hphi, hpsi = q.hv(phi), q.hv(psi)
+        q.close()
+        # a sum of dim terms, and the rounding of H_m phi itself
+        assert abs(g[c] - psi @ hphi) <= 1e-13 * np.linalg.norm(psi) * np.linalg.norm(hphi), channels[c]
+        assert abs(gs[c] - psi @ hpsi) <= 1e-13 * np.linalg.norm(psi) * np.linalg.norm(hpsi), channels[c]
