@@ -99,10 +99,10 @@ __device__ __forceinline__ void sphere_stage(const SphereArgs& a, double*& sF, i
     sLut = tail;
     for (int i = threadIdx.x; i < a.lutSize; i += blockDim.x) sLut[i] = a.lut[(int64_t)i * a.lutStride];
   } else if constexpr (MODE == MODE_RANK_LDS) {
-    sLo = reinterpret_cast<uint32_t*>(tail);
-    sHi = sLo + a.rankLoSize;
-    for (int i = threadIdx.x; i < a.rankLoSize; i += blockDim.x) sLo[i] = a.rankLo[i];
+    sHi = reinterpret_cast<uint32_t*>(tail);
+    sLo16 = reinterpret_cast<uint16_t*>(sHi + a.rankHiSize);
     for (int i = threadIdx.x; i < a.rankHiSize; i += blockDim.x) sHi[i] = a.rankHi[i];
+    for (int i = threadIdx.x; i < a.rankLoSize; i += blockDim.x) sLo16[i] = a.rankLo16[i];
   } else if constexpr (MODE == MODE_RANK_LO16) {
     sLo16 = reinterpret_cast<uint16_t*>(tail);
     sHi = const_cast<uint32_t*>(a.rankHi);
@@ -119,7 +119,7 @@ __device__ __forceinline__ int64_t sphere_find(const SphereArgs& a, uint64_t tgt
                                                const uint32_t* sLo, const uint32_t* sHi, const uint16_t* sLo16) {
   if constexpr (MODE == MODE_BSEARCH)
     return dh_find_bsearch(tgt, sLut, a.lutShift, a.states);
-  else if constexpr (MODE == MODE_RANK_LO16)
+  else if constexpr (MODE == MODE_RANK_LO16 || MODE == MODE_RANK_LDS)
     return dh_find_rank(tgt, sLo16, sHi, a.rankBits, a.dim);
   else
     return dh_find_rank(tgt, sLo, sHi, a.rankBits, a.dim);
@@ -143,7 +143,7 @@ __global__ void __launch_bounds__(1024) sphere_hv_kernel(SphereArgs a, const dou
   constexpr int ROW = ModeRow<MODE>::value;
   // the low table entry: 16-bit copy in LDS (MODE_RANK_LO16), else the 32-bit table (LDS or global)
   auto loAt = [&](uint32_t i) -> uint32_t {
-    if constexpr (BASE == MODE_RANK_LO16)
+    if constexpr (BASE == MODE_RANK_LO16 || BASE == MODE_RANK_LDS)
       return sLo16[i];
     else
       return sLo[i];
@@ -445,16 +445,26 @@ static size_t sphere_lds(const dh_hamiltonian* h, int mode, int lutBitsUsed) {
   size_t bytes = sizeof(double) * h->nbrPackedFactors + sizeof(int) * h->nbrPairSums;
   bytes = (bytes + 7) & ~size_t(7);
   if (mode == MODE_BSEARCH) bytes += sizeof(int) * ((size_t(1) << lutBitsUsed) + 1);
-  if (mode == MODE_RANK_LDS) bytes += sizeof(uint32_t) * (h->basis->rankLoSize + h->basis->rankHiSize);
+  if (mode == MODE_RANK_LDS)
+    bytes += sizeof(uint32_t) * h->basis->rankHiSize + sizeof(uint16_t) * h->basis->rankLoSize;
   if (mode == MODE_RANK_LO16) bytes += sizeof(uint16_t) * h->basis->rankLoSize;
   return bytes;
 }
 
-// where the rank tables of a sphere product are read from (MODE_RANK_LDS, MODE_RANK_LO16 or
-// MODE_RANK_GLOBAL)
-static int sphere_rank_tables(const dh_hamiltonian* h) {
-  if (h->ldsTables && sphere_lds(h, MODE_RANK_LDS, 0) <= 64 * 1024) return MODE_RANK_LDS;
-  if (h->ldsTables && h->basis->d_rankLo16 && sphere_lds(h, MODE_RANK_LO16, 0) <= 96 * 1024) return MODE_RANK_LO16;
+// Where the rank tables of a sphere product of k vectors in workgroups of bs threads are read from:
+// MODE_RANK_LDS (both in LDS), MODE_RANK_LO16 (the low one) or MODE_RANK_GLOBAL.  Both while two workgroups'
+// tables fit a CU (up to 26 orbitals); on 27 and 28 orbitals (82 and 116 KiB) one workgroup of 1024
+// threads can hold them.  The high table's gathers are half of those that bound the product in the L1, and
+// with enough rows to pay the staging that is the better use of the LDS (28 orbitals, 246 k rows: 64.9
+// against 81.8 us, k = 4 191 against 243, k = 8 307 against 381; 723 k rows 284 against 366), except for
+// k = 2, which runs on two lanes per row (102 against 98).  Below 256 rows a CU the staging costs more
+// (62 k rows 29.2 against 28.2, 8 k rows 28.0 against 22.4).
+static int sphere_rank_tables(const dh_hamiltonian* h, int k, int bs) {
+  if (!h->ldsTables || !h->basis->d_rankLo16) return MODE_RANK_GLOBAL;
+  const size_t both = sphere_lds(h, MODE_RANK_LDS, 0);
+  if (both <= 79 * 1024) return MODE_RANK_LDS;
+  if (both <= kLdsLimit && bs == 1024 && k != 2 && h->basis->dim >= (int64_t)h->ctx->nbrCU * 256) return MODE_RANK_LDS;
+  if (sphere_lds(h, MODE_RANK_LO16, 0) <= 96 * 1024) return MODE_RANK_LO16;
   return MODE_RANK_GLOBAL;
 }
 
@@ -497,9 +507,7 @@ template <int K, int LPR>
 static int sphere_dispatch_mode(dh_hamiltonian* h, int bs, const double* x, double* y, int add, int64_t first,
                                 int64_t count) {
   if (h->indexMode == DH_INDEX_BSEARCH) return sphere_launch<K, LPR, MODE_BSEARCH>(h, bs, x, y, add, first, count);
-  // where the rank tables go: both in LDS when they fit 64 KiB, else the 16-bit low table in LDS
-  // (the high table from L2), else both from global memory
-  const int where = sphere_rank_tables(h);
+  const int where = sphere_rank_tables(h, K, bs);
   const bool tablesInLds = where == MODE_RANK_LDS, lo16 = where == MODE_RANK_LO16;
   if (h->indexMode == DH_INDEX_RANK_X4) {
     if (tablesInLds) return sphere_launch<K, LPR, MODE_RANK_LDS_X4>(h, bs, x, y, add, first, count);
@@ -524,7 +532,7 @@ static int sphere_dispatch_lpr(dh_hamiltonian* h, const double* x, double* y, in
                                int64_t count) {
   int lpr = h->lanesPerRow, bs = h->blockSize;
   if (h->autoLaunch) {
-    // the fastest shapes measured on MI355X by rows per CU and k, times in us.  Few rows: lanes for
+    // the fastest shapes measured on MI355X by rows per CU and k, times in us (the high table in L2).  Few rows: lanes for
     // wavefronts, in small workgroups (338 rows: 9.1 with 2 x 256, 10.2 with 4 x 512; 45 k rows: 26.2 with
     // 2 x 512, 36.8 with 4 x 512; 71 k rows: 37.9 with 1 x 512, 53 with 1 x 1024 and 2 x 256, k = 4 81 with
     // 2 x 1024, 110 and more with one lane; k = 8, 8512 rows: 23.3 with 8 x 256, 31.8 with 4 x 512).  Many
@@ -539,7 +547,7 @@ static int sphere_dispatch_lpr(dh_hamiltonian* h, const double* x, double* y, in
       K <= 2 ? set(2, 256) : set(8, 256);
     else if (perCU < 256)
       K <= 2 ? set(2, 512) : set(4, 1024);
-    else if (sphere_rank_tables(h) == MODE_RANK_GLOBAL)
+    else if (sphere_rank_tables(h, K, 1024) == MODE_RANK_GLOBAL)
       set(2, K <= 2 ? 256 : 1024);
     else if (K == 1)
       set(1, perCU < 512 ? 512 : 1024);

@@ -335,7 +335,9 @@ __device__ __forceinline__ int tile_sector(const int64_t* sPrefix, int nActive, 
 // 32-bit in both forms.
 // FREE: the created pairs come from the set bits of the free-pair masks (dh_sphere_row).
 // TRI: the factor matrices are triangles (dh_pack_sphere_factors).
-template <int K, int LPR, bool LO_LDS, bool S32, bool FREE, bool TRI>
+// TABLES: the rank tables in LDS: 0 none, 1 the low one (16 bits), 2 the sector's high one too, staged when
+// a workgroup's tiles enter a sector.
+template <int K, int LPR, int TABLES, bool S32, bool FREE, bool TRI>
 __global__ void __launch_bounds__(1024) sectors_hv_kernel(SectorsArgs a, const double* __restrict__ x,
                                                           double* __restrict__ y, int add) {
   extern __shared__ double smem[];
@@ -346,12 +348,14 @@ __global__ void __launch_bounds__(1024) sectors_hv_kernel(SectorsArgs a, const d
   for (int i = threadIdx.x; i < a.nbrFactors; i += blockDim.x) sF[i] = a.factors[i];
   for (int i = threadIdx.x; i < a.nbrSums; i += blockDim.x) sBase[i] = a.sumBase[i];
   for (int i = threadIdx.x; i < 2 * a.nActive + 1; i += blockDim.x) sWork[i] = a.work[i];
-  if constexpr (LO_LDS)
+  uint32_t* sHi = reinterpret_cast<uint32_t*>(sLo + a.loSize);
+  if constexpr (TABLES > 0)
     for (int i = threadIdx.x; i < a.loSize; i += blockDim.x) sLo[i] = a.rankLo16[i];
   __syncthreads();
+  int staged = -1;  // the sector whose high table is in LDS
   // the low table: 16-bit copy in LDS, or the 32-bit table in global memory
   auto loAt = [&](uint32_t i) -> uint32_t {
-    if constexpr (LO_LDS)
+    if constexpr (TABLES > 0)
       return sLo[i];
     else
       return a.rankLo[i];
@@ -362,9 +366,21 @@ __global__ void __launch_bounds__(1024) sectors_hv_kernel(SectorsArgs a, const d
   for (int64_t tile = dh_xcd_block(blockIdx.x, gridDim.x); tile < a.totalTiles; tile += gridDim.x) {
     const int j = tile_sector(sPrefix, a.nActive, tile);
     const int sec = (int)sWork[j];
+    if constexpr (TABLES == 2) {
+      if (sec != staged) {
+        __syncthreads();  // the last tile's lookups are done
+        for (int i = threadIdx.x; i < a.hiSize; i += blockDim.x) sHi[i] = a.rankHi[(int64_t)sec * a.hiSize + i];
+        __syncthreads();
+        staged = sec;
+      }
+    }
     const int64_t off = a.offsets[sec];
     const int64_t dim = a.offsets[sec + 1] - off;
-    const uint32_t* hi = a.rankHi + (int64_t)sec * a.hiSize;
+    const uint32_t* hi;
+    if constexpr (TABLES == 2)
+      hi = sHi;
+    else
+      hi = a.rankHi + (int64_t)sec * a.hiSize;
     const int64_t local = (tile - sPrefix[j]) * rowsPerTile + threadIdx.x / LPR;
     const bool active = local < dim;
     const int64_t g = off + (active ? local : 0);
@@ -426,13 +442,24 @@ static SectorsArgs sectors_args(dh_sector_set* S, int nActive, int64_t totalTile
   return a;
 }
 
-// Dynamic LDS for `na` active sectors: the packed factors and the work list, with the 16-bit low rank
-// table when it exists and two workgroups' tables fit a CU's 160 KiB.
-static size_t sectors_lds(const dh_sector_set* S, int na, bool* loLds) {
+// Dynamic LDS for `na` active sectors and workgroups of bs threads: the packed factors and the work list,
+// with the rank tables that go there (TABLES of the kernel): the low one while two workgroups' tables fit a
+// CU, and the high one too while two still fit (up to 26 orbitals) or one that fills the CU (27 and 28
+// orbitals, 1024 threads).  The high table's gathers are half of those that bound the product in the L1:
+// 1.0 M rows on 25 orbitals 214 -> 201 us, k = 8 948 -> 811; 6.7 M rows on 28 orbitals 1595 -> 1549 us, k = 2
+// 2228 -> 1706, k = 8 8605 -> 7032.
+static size_t sectors_lds(const dh_sector_set* S, int na, int bs, int* tables) {
   const size_t base = ((size_t)S->nbrPackedFactors * 8 + (size_t)S->nbrPairSums * 4 + 7) / 8 * 8 + 8 * (2 * na + 1);
-  const size_t withLo = base + 2 * S->loSize;
-  *loLds = S->d_rankLo16 && withLo <= 79 * 1024;
-  return *loLds ? withLo : base;
+  const size_t lo = base + 2 * S->loSize, both = lo + 4 * S->hiSize;
+  *tables = 0;
+  if (!S->d_rankLo16) return base;
+  if (both <= 79 * 1024 || (both <= 160 * 1024 && bs == 1024)) {
+    *tables = 2;
+    return both;
+  }
+  if (lo > 79 * 1024) return base;
+  *tables = 1;
+  return lo;
 }
 
 template <int K, int LPR>
@@ -445,8 +472,8 @@ static int sectors_hv_launch(dh_sector_set* S, int blockSize, const double* x, d
   int rc = dh_sectors_upload_work(S, active, rowsPerTile, &na, &tiles);
   if (rc) return rc;
   if (tiles == 0) return DH_OK;
-  bool loLds;
-  const size_t lds = sectors_lds(S, na, &loLds);
+  int tables;
+  const size_t lds = sectors_lds(S, na, blockSize, &tables);
   if (lds > 160 * 1024) return dh_fail(c, DH_E_RANGE, "staged tables exceed LDS");
   SectorsArgs a = sectors_args(S, na, tiles);
   auto launch = [&](auto kern) -> int {
@@ -466,26 +493,32 @@ static int sectors_hv_launch(dh_sector_set* S, int blockSize, const double* x, d
   // MI355X, as for a single space)
   const bool freePairs = S->rowMode == DH_INDEX_RANK_FREE || (S->rowMode == DH_INDEX_RANK && K <= 2);
   auto pick = [&](auto lo, auto tri) -> int {
-    constexpr bool LO = decltype(lo)::value, TRI = decltype(tri)::value;
+    constexpr int LO = decltype(lo)::value;
+    constexpr bool TRI = decltype(tri)::value;
     if (freePairs)
       return s32 ? launch(sectors_hv_kernel<K, LPR, LO, (K <= 2), true, TRI>)
                  : launch(sectors_hv_kernel<K, LPR, LO, false, true, TRI>);
     return s32 ? launch(sectors_hv_kernel<K, LPR, LO, (K <= 2), false, TRI>)
                : launch(sectors_hv_kernel<K, LPR, LO, false, false, TRI>);
   };
-  if (S->triangles) return loLds ? pick(std::true_type{}, std::true_type{}) : pick(std::false_type{}, std::true_type{});
-  return loLds ? pick(std::true_type{}, std::false_type{}) : pick(std::false_type{}, std::false_type{});
+  auto where = [&](auto tri) -> int {
+    switch (tables) {
+      case 0: return pick(std::integral_constant<int, 0>{}, tri);
+      case 1: return pick(std::integral_constant<int, 1>{}, tri);
+      default: return pick(std::integral_constant<int, 2>{}, tri);
+    }
+  };
+  return S->triangles ? where(std::true_type{}) : where(std::false_type{});
 }
 
-// Lanes per row and workgroup size by rows per CU and k, times in us on MI355X (the set's default was
-// 1 x 256).  Few rows: lanes for wavefronts (26 k rows: 20.1 with 2 x 256, 22.9; 4173 rows, k = 4: 16.7
-// with 8 x 256, 33.0).  To 2048 rows a CU small workgroups spread best (164 k rows: 39.7 with 1 x 256,
-// 45 with 1 x 512 and 1 x 1024; k = 4: 80 with 2 x 256, 96 with 1 x 256).  Above, the tables in LDS bound
-// the wavefronts of a CU: 512 threads when three workgroups fit it, else 1024 (1.0 M rows: 205 and 215,
-// 248 at 256; 17.6 M rows with 29 orbitals, two workgroups: 5.4 ms at 1024, 8.4 at 512, 14.0 at 256;
-// k = 4, 6.7 M rows, three: 4.7 ms at 512, 6.5 at 1024, 8.1 at 256).  k = 8 and 16: two lanes, 512 (1.0 M
-// rows 943 against 1012 and 2178 against 2934), except k = 8 with many rows (6.7 M: 8.6 ms with 1 x 1024,
-// 9.5 with 2 x 512).
+// Lanes per row and workgroup size by rows per CU and k, times in us on MI355X.  Few rows: lanes for
+// wavefronts (26 k rows: 19.0 with 2 x 256, 21.5 with 1 x 256; 4173 rows, k = 4: 16.7 with 8 x 256, 33.0).
+// To 2048 rows a CU small workgroups spread best (164 k rows: 35.4 with 1 x 256, 40 with 1 x 512 and
+// 1 x 1024; k = 4: 73 with 2 x 256, 85 with 1 x 256).  Above, the tables in LDS bound the wavefronts of a
+// CU: 1024 threads (1.0 M rows: 188, 232 at 256; 17.6 M rows with 29 orbitals: 5.4 ms, 8.4 at 512, 14.0 at
+// 256), for k = 4 512 when three workgroups fit (1.0 M rows, 25 orbitals: 432, 523 at 1024).  k = 8 and 16:
+// two lanes, 512 (1.0 M rows 810 against 861 and 2143 against 2295 at 2 x 1024), except k = 8 with many rows
+// (6.7 M: 7.0 ms with 1 x 1024, 9.5 with 2 x 512).
 static void sectors_shape(const dh_sector_set* S, int k, int* lpr, int* bs) {
   *lpr = S->lanesPerRow;
   *bs = S->blockSize;
@@ -495,10 +528,10 @@ static void sectors_shape(const dh_sector_set* S, int k, int* lpr, int* bs) {
   if (perCU < 128) return k <= 2 ? set(2, 256) : set(8, 256);
   if (perCU < 2048) return k <= 2 ? set(1, 256) : set(2, 256);
   if (k > 8 || (k == 8 && perCU < 8192)) return set(2, 512);
-  bool lo;
-  const bool three = 3 * sectors_lds(S, S->nbrSectors, &lo) <= 160 * 1024;
-  if (k == 8 || !three || (k <= 2 && perCU >= 8192)) return set(1, 1024);
-  set(1, 512);
+  int tables;
+  const bool oneFills = sectors_lds(S, S->nbrSectors, 1024, &tables) > 79 * 1024 && tables == 2;
+  const bool three = 3 * sectors_lds(S, S->nbrSectors, 512, &tables) <= 160 * 1024;
+  k == 4 && three && !oneFills ? set(1, 512) : set(1, 1024);
 }
 
 template <int K>

@@ -300,3 +300,23 @@ def test_large_sectors_run_alone_in_a_batched_solve(arch, golden, k):
         np.testing.assert_allclose(ea[i, :m], es[i, :m], rtol=0, atol=1e-10)
     ref = np.array(golden["fermions_sphere_n8_2s21_lz0"]["eigenvalues"])
     np.testing.assert_allclose(ea[0], ref, rtol=0, atol=1e-10)
+
+
+# the sector's high rank table in LDS: up to 26 orbitals in any workgroup, on 27 and 28 in one of 1024
+# threads, restaged as the workgroup's tiles pass from sector to sector; 29 orbitals never
+@pytest.mark.parametrize("n,lz,lpr,block", [(4, 25, 1, 256), (4, 26, 2, 1024), (4, 27, 1, 1024), (4, 27, 1, 512),
+                                            (4, 28, 1, 1024), (3, 27, 0, 0)])
+@pytest.mark.parametrize("k", [1, 2, 4, 16])
+def test_rank_tables_in_lds_match_single_spaces(arch, n, lz, lpr, block, k):
+    V = coulomb(lz)
+    sectors = [s for s in range((n * lz) % 2, 60, 2)]
+    S = SectorSet(arch, n, lz, sectors, V)
+    if lpr:
+        assert S.capi.gpu().dh_sector_set_launch(S.h, lpr, block) == 0
+    X = np.random.default_rng(lz + k).standard_normal((S.total, k))
+    Y = S.hv(X.reshape(-1), k).reshape(S.total, k)
+    for i, total_lz in enumerate(sectors):
+        a, b = S.off[i], S.off[i + 1]
+        ref = O.fs_hv(O.FermionSphere(n, total_lz, lz), O.Factors(lz, V), np.ascontiguousarray(X[a:b, 0]))
+        assert np.linalg.norm(Y[a:b, 0] - ref) <= 1e-12 * np.linalg.norm(ref), (total_lz, k)
+    S.close()

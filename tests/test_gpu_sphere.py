@@ -432,3 +432,18 @@ def test_basis_from_diagham_states(arch):
     assert capi.gpu().dh_fermion_sphere_from_states(arch.ctx, ctypes.byref(bad), n, lz, lz_max,
                                                     words.ctypes.data_as(capi.P_U64), words.size - 1) == capi.DH_E_ARG
     assert b"not the full sector" in capi.gpu().dh_last_error(arch.ctx)
+
+
+@pytest.mark.parametrize("n,total_lz,lz", [(10, 0, 27), (10, 4, 26)])
+@pytest.mark.parametrize("k", [1, 4])
+def test_both_rank_tables_in_lds(arch, n, total_lz, lz, k):
+    """27 and 28 orbitals with enough rows: 1024-thread workgroups hold both rank tables."""
+    from diagham_amd import capi
+    V = capi.coulomb_pseudopotentials(lz, True)
+    p = capi.Problem.sphere(arch, n, total_lz, lz, V)
+    assert p.dim >= 65536 * 2
+    X = np.random.default_rng(k).standard_normal((p.dim, k))
+    Y = p.hv(X.reshape(-1), k).reshape(p.dim, k)
+    p.close()
+    ref = O.fs_hv(O.FermionSphere(n, total_lz, lz), O.Factors(lz, V), np.ascontiguousarray(X[:, k - 1]))
+    assert np.linalg.norm(Y[:, k - 1] - ref) <= 1e-12 * np.linalg.norm(ref)
