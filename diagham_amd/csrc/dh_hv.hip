@@ -504,8 +504,8 @@ static int sphere_launch(dh_hamiltonian* h, int bs, const double* x, double* y, 
 }
 
 template <int K, int LPR>
-static int sphere_dispatch_mode(dh_hamiltonian* h, int bs, const double* x, double* y, int add, int64_t first,
-                                int64_t count) {
+static int sphere_dispatch_mode(dh_hamiltonian* h, int bs, bool freePairs, const double* x, double* y, int add,
+                                int64_t first, int64_t count) {
   if (h->indexMode == DH_INDEX_BSEARCH) return sphere_launch<K, LPR, MODE_BSEARCH>(h, bs, x, y, add, first, count);
   const int where = sphere_rank_tables(h, K, bs);
   const bool tablesInLds = where == MODE_RANK_LDS, lo16 = where == MODE_RANK_LO16;
@@ -514,9 +514,6 @@ static int sphere_dispatch_mode(dh_hamiltonian* h, int bs, const double* x, doub
     if (lo16) return sphere_launch<K, LPR, MODE_RANK_LO16_X4>(h, bs, x, y, add, first, count);
     return sphere_launch<K, LPR, MODE_RANK_GLOBAL_X4>(h, bs, x, y, add, first, count);
   }
-  // DH_INDEX_RANK: the free-pair masks for k <= 2 (fewer instructions per term), the range loop for
-  // k > 2 (where the masks' extra registers cost more than they save)
-  const bool freePairs = h->indexMode == DH_INDEX_RANK_FREE || (h->indexMode == DH_INDEX_RANK && K <= 2);
   if (freePairs) {
     if (tablesInLds) return sphere_launch<K, LPR, MODE_RANK_LDS_FREE>(h, bs, x, y, add, first, count);
     if (lo16) return sphere_launch<K, LPR, MODE_RANK_LO16_FREE>(h, bs, x, y, add, first, count);
@@ -531,42 +528,59 @@ template <int K>
 static int sphere_dispatch_lpr(dh_hamiltonian* h, const double* x, double* y, int add, int64_t first,
                                int64_t count) {
   int lpr = h->lanesPerRow, bs = h->blockSize;
+  // DH_INDEX_RANK in a chosen shape: the free-pair masks for k <= 2 and the range loop above, so that more than
+  // two vectors give the same bits in every grouping; in an automatic one the faster of the two, the masks
+  // (fewer instructions per term) up to k = 8 (1.4 M rows 2.2 against 2.8 ms), for k = 16 the range loop, where
+  // their registers cost more than they save (7.5 against 6.4)
+  bool freePairs = h->indexMode == DH_INDEX_RANK_FREE || (h->indexMode == DH_INDEX_RANK && K <= (h->autoLaunch ? 8 : 2));
   if (h->autoLaunch) {
-    // the fastest shapes measured on MI355X by rows per CU and k, times in us (the high table in L2).  Few rows: lanes for
-    // wavefronts, in small workgroups (338 rows: 9.1 with 2 x 256, 10.2 with 4 x 512; 45 k rows: 26.2 with
-    // 2 x 512, 36.8 with 4 x 512; 71 k rows: 37.9 with 1 x 512, 53 with 1 x 1024 and 2 x 256, k = 4 81 with
-    // 2 x 1024, 110 and more with one lane; k = 8, 8512 rows: 23.3 with 8 x 256, 31.8 with 4 x 512).  Many
-    // rows: with the 16-bit low table in LDS a workgroup holds about 60 KiB, two per CU, so 1024 threads
-    // (1.4 M rows: 603, 645 at 512; k = 4: 1436, 2068 at 512).  k = 8 and 16 wait for their 64- and
-    // 128-byte gathers: two lanes (1.4 M rows: 2838 against 2898 and 6450 against 7300), and k = 8 one lane
-    // and 512 threads past 8192 rows a CU (7.8 M rows: 20.7 ms against 22.5).  With both tables in global
-    // memory: two lanes per row, 256 threads for k <= 2, 1024 above.
+    // The fastest shapes measured on MI355X by rows per CU and k, times in us.  Few rows: eight lanes, whose
+    // rows finish together with the range loop (338 rows: 7.7, 9.2 with 2 x 256 and the masks; 13 k rows 18.9
+    // and 20.6; k = 8 15.9 and 17.7).  Then lanes for wavefronts in small workgroups (45 k rows: 26.2 with
+    // 2 x 512, 36.8 with 4 x 512; k = 4 37.0 with 2 x 512, 43.1 by ranges; k = 8 50.7 with 4 x 256; 71 k rows:
+    // 37.9 with 1 x 512, 53 with 1 x 1024; k = 4 54.9 with 2 x 1024).  Many rows: the tables in LDS leave two
+    // workgroups a CU or one, so 1024 threads (1.4 M rows: 603, 645 at 512); with the high table in L2 (not
+    // both in LDS) k = 4 and 8 run better on fewer wavefronts (1.4 M rows: 1377 with 1 x 512, 1436 at 1024, and
+    // 2200 with 2 x 512, 2265 at 1024; 246 k rows, both in LDS: 134 with 1 x 1024, 171 at 512, and 271 with
+    // 2 x 1024, 301 at 512), past 8192 rows a CU k = 2 too (7.8 M rows: 6.4 ms with 2 x 512, 7.1 at 1024; k = 8
+    // 19.1 with 1 x 512, 19.7 with 2).  With both tables in global memory: two lanes per row, 256 threads for
+    // k <= 2, 1024 above.
     const int64_t perCU = h->basis->dim / h->ctx->nbrCU;
+    const int tables = sphere_rank_tables(h, K, 1024);
     auto set = [&](int l, int b) { lpr = l, bs = b; };
-    if (perCU < 64)
-      K <= 2 ? set(2, 256) : set(8, 256);
-    else if (perCU < 256)
-      K <= 2 ? set(2, 512) : set(4, 1024);
-    else if (sphere_rank_tables(h, K, 1024) == MODE_RANK_GLOBAL)
+    if (perCU < 64) {
+      set(8, 256);
+      freePairs = false;
+    } else if (perCU < 256) {
+      K <= 4 ? set(2, 512) : set(4, 256);
+      freePairs = true;
+    } else if (tables == MODE_RANK_GLOBAL) {
       set(2, K <= 2 ? 256 : 1024);
-    else if (K == 1)
-      set(1, perCU < 512 ? 512 : 1024);
-    else if (K == 4 && perCU >= 512)
+      freePairs = K <= 2;
+    } else if (perCU < 512) {
+      K == 1 ? set(1, 512) : K == 16 ? set(8, 256) : set(2, 1024);
+      freePairs = true;
+    } else if (K == 1) {
       set(1, 1024);
-    else if (K == 8 && perCU >= 8192)
-      set(1, 512);
-    else
+    } else if (K == 2) {
+      set(2, perCU < 8192 ? 1024 : 512);
+    } else if (K == 4) {
+      set(1, tables == MODE_RANK_LDS ? 1024 : 512);
+    } else if (K == 8 && tables != MODE_RANK_LDS) {
+      set(perCU < 8192 ? 2 : 1, 512);
+    } else {
       set(2, 1024);
+    }
   }
   // k = 2 with one lane per row faulted the GPU twice on N=5 2S=33 (free-pair rows, with the low
   // rank table in LDS and in global memory) with no cause found in the code; k = 2 runs with two
   // lanes per row, as tested, until one is
   if (K == 2 && lpr == 1) lpr = 2;
   switch (lpr) {
-    case 1: return sphere_dispatch_mode<K, 1>(h, bs, x, y, add, first, count);
-    case 2: return sphere_dispatch_mode<K, 2>(h, bs, x, y, add, first, count);
-    case 4: return sphere_dispatch_mode<K, 4>(h, bs, x, y, add, first, count);
-    case 8: return sphere_dispatch_mode<K, 8>(h, bs, x, y, add, first, count);
+    case 1: return sphere_dispatch_mode<K, 1>(h, bs, freePairs, x, y, add, first, count);
+    case 2: return sphere_dispatch_mode<K, 2>(h, bs, freePairs, x, y, add, first, count);
+    case 4: return sphere_dispatch_mode<K, 4>(h, bs, freePairs, x, y, add, first, count);
+    case 8: return sphere_dispatch_mode<K, 8>(h, bs, freePairs, x, y, add, first, count);
     default: return dh_fail(h->ctx, DH_E_ARG, "lanes_per_row must be 1, 2, 4 or 8 for this Hamiltonian");
   }
 }

@@ -463,7 +463,7 @@ static size_t sectors_lds(const dh_sector_set* S, int na, int bs, int* tables) {
 }
 
 template <int K, int LPR>
-static int sectors_hv_launch(dh_sector_set* S, int blockSize, const double* x, double* y, int add,
+static int sectors_hv_launch(dh_sector_set* S, int blockSize, bool freePairs, const double* x, double* y, int add,
                              const unsigned char* active) {
   dh_context* c = S->ctx;
   int64_t rowsPerTile = blockSize / LPR;
@@ -489,9 +489,6 @@ static int sectors_hv_launch(dh_sector_set* S, int blockSize, const double* x, d
   // more vectors the 64-bit form is faster on MI355X (its lower occupancy keeps more of the x
   // gathers in cache: 11.3 against 16.5 ms at k = 8 over the 91 sectors of N=10 2S=27)
   const bool s32 = K <= 2 && S->nbrOrbitals <= 32;
-  // DH_INDEX_RANK: the free-pair masks for k <= 2, the range loop for k > 2 (the faster per k on
-  // MI355X, as for a single space)
-  const bool freePairs = S->rowMode == DH_INDEX_RANK_FREE || (S->rowMode == DH_INDEX_RANK && K <= 2);
   auto pick = [&](auto lo, auto tri) -> int {
     constexpr int LO = decltype(lo)::value;
     constexpr bool TRI = decltype(tri)::value;
@@ -511,38 +508,60 @@ static int sectors_hv_launch(dh_sector_set* S, int blockSize, const double* x, d
   return S->triangles ? where(std::true_type{}) : where(std::false_type{});
 }
 
-// Lanes per row and workgroup size by rows per CU and k, times in us on MI355X.  Few rows: lanes for
-// wavefronts (26 k rows: 19.0 with 2 x 256, 21.5 with 1 x 256; 4173 rows, k = 4: 16.7 with 8 x 256, 33.0).
-// To 2048 rows a CU small workgroups spread best (164 k rows: 35.4 with 1 x 256, 40 with 1 x 512 and
-// 1 x 1024; k = 4: 73 with 2 x 256, 85 with 1 x 256).  Above, the tables in LDS bound the wavefronts of a
-// CU: 1024 threads (1.0 M rows: 188, 232 at 256; 17.6 M rows with 29 orbitals: 5.4 ms, 8.4 at 512, 14.0 at
-// 256), for k = 4 512 when three workgroups fit (1.0 M rows, 25 orbitals: 432, 523 at 1024).  k = 8 and 16:
-// two lanes, 512 (1.0 M rows 810 against 861 and 2143 against 2295 at 2 x 1024), except k = 8 with many rows
-// (6.7 M: 7.0 ms with 1 x 1024, 9.5 with 2 x 512).
-static void sectors_shape(const dh_sector_set* S, int k, int* lpr, int* bs) {
+// Lanes per row, workgroup size and row routine by rows per CU and k, times in us on MI355X.  Few rows: eight
+// lanes and the range loop, whose rows finish together (4173 rows: 14.7, 15.7 with 2 x 256 and the masks; k = 4
+// 16.8 and 17.8).  Then lanes for wavefronts (26 k rows: 19.3 with 2 x 256, 21.5 with 1 x 256; k = 16 43.5 with
+// 4 x 256, 49.9 with 2).  From 128 to 2048 rows a CU small workgroups spread best (164 k rows: 35.4 with
+// 1 x 256, 40 with 1 x 512 and 1 x 1024; k = 4: 55 with 2 x 256, 60 with 1 x 512, 71 by ranges; k = 8: 99, 125
+// by ranges; k = 16: 285 with 4 x 256, 375 with 2 x 512 by ranges).  Above, the tables in LDS bound the
+// wavefronts of a CU: 1024 threads (1.0 M rows: 188, 232 at 256; 17.6 M rows with 29 orbitals: 5.4 ms, 8.4 at
+// 512, 14.0 at 256), for k = 4 512 when three workgroups fit (1.0 M rows, 25 orbitals: 314, 336 at 1024, 425 by
+// ranges).  k = 8: two lanes, 1024 threads where one workgroup's tables fill a CU (6.7 M rows: 6.0 ms, 7.0 with
+// 2 x 512), 512 where more fit (1.0 M rows: 676, 725 at 1024), one lane with the high table in L2 (17.6 M rows
+// 22.3 ms, 23.7 with two).  k = 16: two lanes, 512, and by ranges (2139, 2242 with the masks).
+static void sectors_shape(const dh_sector_set* S, int k, int* lpr, int* bs, bool* freePairs) {
   *lpr = S->lanesPerRow;
   *bs = S->blockSize;
+  // DH_INDEX_RANK in a chosen shape: the free-pair masks for k <= 2, as for a single space
+  *freePairs = S->rowMode == DH_INDEX_RANK_FREE || (S->rowMode == DH_INDEX_RANK && k <= 2);
   if (!S->autoLaunch) return;
   const int64_t perCU = S->totalDim / S->ctx->nbrCU;
+  bool masks = true;
   auto set = [&](int l, int b) { *lpr = l, *bs = b; };
-  if (perCU < 128) return k <= 2 ? set(2, 256) : set(8, 256);
-  if (perCU < 2048) return k <= 2 ? set(1, 256) : set(2, 256);
-  if (k > 8 || (k == 8 && perCU < 8192)) return set(2, 512);
-  int tables;
-  const bool oneFills = sectors_lds(S, S->nbrSectors, 1024, &tables) > 79 * 1024 && tables == 2;
-  const bool three = 3 * sectors_lds(S, S->nbrSectors, 512, &tables) <= 160 * 1024;
-  k == 4 && three && !oneFills ? set(1, 512) : set(1, 1024);
+  if (perCU < 32) {
+    set(8, 256);
+    masks = false;
+  } else if (perCU < 128) {
+    set(k == 16 ? 4 : 2, 256);
+  } else if (perCU < 2048) {
+    set(k <= 2 ? 1 : k == 16 ? 4 : 2, 256);
+  } else if (k == 16) {
+    set(2, 512);
+    masks = false;
+  } else {
+    int tables;
+    const bool three = 3 * sectors_lds(S, S->nbrSectors, 512, &tables) <= 160 * 1024;
+    const bool oneFills = sectors_lds(S, S->nbrSectors, 1024, &tables) > 79 * 1024 && tables == 2;
+    if (k <= 2)
+      set(1, 1024);
+    else if (k == 4)
+      set(1, three && !oneFills ? 512 : 1024);
+    else
+      oneFills ? set(2, 1024) : set(tables == 2 ? 2 : 1, 512);
+  }
+  if (S->rowMode == DH_INDEX_RANK) *freePairs = masks;
 }
 
 template <int K>
 static int sectors_hv_lpr(dh_sector_set* S, const double* x, double* y, int add, const unsigned char* active) {
   int lpr, bs;
-  sectors_shape(S, K, &lpr, &bs);
+  bool freePairs;
+  sectors_shape(S, K, &lpr, &bs, &freePairs);
   switch (lpr) {
-    case 1: return sectors_hv_launch<K, 1>(S, bs, x, y, add, active);
-    case 2: return sectors_hv_launch<K, 2>(S, bs, x, y, add, active);
-    case 4: return sectors_hv_launch<K, 4>(S, bs, x, y, add, active);
-    default: return sectors_hv_launch<K, 8>(S, bs, x, y, add, active);
+    case 1: return sectors_hv_launch<K, 1>(S, bs, freePairs, x, y, add, active);
+    case 2: return sectors_hv_launch<K, 2>(S, bs, freePairs, x, y, add, active);
+    case 4: return sectors_hv_launch<K, 4>(S, bs, freePairs, x, y, add, active);
+    default: return sectors_hv_launch<K, 8>(S, bs, freePairs, x, y, add, active);
   }
 }
 

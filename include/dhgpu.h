@@ -42,8 +42,8 @@ typedef struct dh_hamiltonian dh_hamiltonian;
 /* index lookup used by the H.v kernels */
 #define DH_INDEX_BSEARCH 0 /* top-bit LUT staged in LDS, then binary search of the sorted basis */
 #define DH_INDEX_RANK 1    /* combinatorial rank: two table lookups, no basis probes; on the sphere
-                              the two-body created pairs come from the free-pair masks for k <= 2
-                              and from the range loop for k > 2, the faster of the two per k */
+                              the two-body created pairs come from the free-pair masks or the range
+                              loop, the faster of the two by k and the number of rows */
 #define DH_INDEX_RANK_X4 2 /* rank, with the two-body created-pair loop unrolled four-wide (sphere only;
                               other Hamiltonians treat it as DH_INDEX_RANK) */
 #define DH_INDEX_RANK_FREE 3 /* rank, with the created pairs taken from the mask of free pairs of each
@@ -214,8 +214,8 @@ int dh_sector_set_factors(dh_sector_set* set, const double* factors, const int* 
 int dh_sector_set_launch(dh_sector_set* set, int lanes_per_row, int block_size);
 /* Row routine of the products of a sphere or momentum set: DH_INDEX_RANK_RANGE (every created pair
  * of the range or list, skipping occupied ones), DH_INDEX_RANK_FREE (only the free created pairs,
- * from one bit mask per annihilated pair) or DH_INDEX_RANK (sphere sets: free pairs for k <= 2, the
- * range for k > 2; momentum sets: the list).  A tuning knob like dh_sector_set_launch; the results
+ * from one bit mask per annihilated pair) or DH_INDEX_RANK (sphere sets: the faster of the two by k
+ * and the number of rows; momentum sets: the free pairs).  A tuning knob like dh_sector_set_launch; the results
  * agree to rounding. */
 int dh_sector_set_row_mode(dh_sector_set* set, int mode);
 /* Launch shape of the segmented vector operations of a set (no counterpart in the reference, a
