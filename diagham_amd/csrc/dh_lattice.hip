@@ -380,7 +380,8 @@ struct LatticeTables {  // LDS
 // accesses each per wavefront.  With the factors in LDS the L1 has two thirds of them (41 M of 55 M cycles a
 // CU; 62 M of 74 M without).  32-bit words (up to 32 orbitals) take 30 vector instructions a term, 60 with a
 // free mask per intermediate state and popcounts on 64-bit words.  30 sectors of 10 fermions on 6 x 5 sites:
-// 46.4 ms so, 31.0 with these masks, 23.5 with the factors in LDS.
+// 46.4 ms so, 31.0 with these masks, 23.5 with the factors in LDS.  HI_LDS: the sector's high rank table there
+// too, the other gather that is not x.
 template <int K, int LPR, typename U, typename Find>
 __device__ __forceinline__ void lattice_row_free(U s, int N, int ny, const LatticeTables& T,
                                                  const double2* factors, int lane, Find find,
@@ -465,7 +466,7 @@ __device__ __forceinline__ void lattice_row_free(U s, int N, int ny, const Latti
 // K complex vectors per row: x and y hold 2K doubles per row, (re, im) interleaved.  ROWS: 0, every
 // listed pair of the momentum sum is tried; 32 and 64, the free-pair masks (lattice_row_free) on words
 // of that many bits.
-template <int K, int LPR, bool LO_LDS, int ROWS, bool FAC_LDS>
+template <int K, int LPR, bool LO_LDS, int ROWS, bool FAC_LDS, bool HI_LDS = false>
 __global__ void __launch_bounds__(1024) lattice_hv_kernel(LatticeArgs a, const double* __restrict__ x,
                                                           double* __restrict__ y, int add) {
   constexpr bool FREE = ROWS != 0;
@@ -506,9 +507,11 @@ __global__ void __launch_bounds__(1024) lattice_hv_kernel(LatticeArgs a, const d
   if constexpr (FAC_LDS)
     for (int i = threadIdx.x; i < a.nbrFactors; i += blockDim.x)
       sFac[i] = reinterpret_cast<const double2*>(a.factors)[i];
+  uint32_t* sHi = reinterpret_cast<uint32_t*>(sLo + a.loSize);  // HI_LDS: hiSize
   if constexpr (LO_LDS)
     for (int i = threadIdx.x; i < a.loSize; i += blockDim.x) sLo[i] = a.rankLo16[i];
   __syncthreads();
+  int staged = -1;  // the sector whose high table is in LDS
   const LoT* lo;
   if constexpr (LO_LDS)
     lo = sLo;
@@ -522,7 +525,18 @@ __global__ void __launch_bounds__(1024) lattice_hv_kernel(LatticeArgs a, const d
     const int sec = (int)sWork[j];
     const int64_t off = a.offsets[sec];
     const int64_t dim = a.offsets[sec + 1] - off;
-    const uint32_t* hi = a.rankHi + (int64_t)sec * a.hiSize;
+    const uint32_t* hi;
+    if constexpr (HI_LDS) {
+      if (sec != staged) {
+        __syncthreads();  // the last tile's lookups are done
+        for (int i = threadIdx.x; i < a.hiSize; i += blockDim.x) sHi[i] = a.rankHi[(int64_t)sec * a.hiSize + i];
+        __syncthreads();
+        staged = sec;
+      }
+      hi = sHi;
+    } else {
+      hi = a.rankHi + (int64_t)sec * a.hiSize;
+    }
     const int64_t local = (tile - sPrefix[j]) * rowsPerTile + threadIdx.x / LPR;
     const bool active = local < dim;
     const int64_t g = off + (active ? local : 0);
@@ -629,6 +643,10 @@ struct LatticeLds {
   bool free;  // DH_INDEX_RANK: the free-pair masks
   size_t tables, withLo, withFactors;
   bool factorsFit;  // one workgroup of a CU can hold all of it (32-bit words only: 30 orbitals take 147 KiB)
+  // and the sector's high rank table, staged when the workgroup's tiles enter a sector (up to 27 orbitals:
+  // 735 k rows on 24 orbitals 271 -> 201 us, k = 2 346 -> 272, k = 8 1928 -> 1785; 2.2 M rows on 27 777 -> 674)
+  size_t withHi;
+  bool hiFits;
 };
 
 static LatticeLds lattice_lds(const dh_sector_set* S, int na) {
@@ -650,6 +668,8 @@ static LatticeLds lattice_lds(const dh_sector_set* S, int na) {
   l.withLo = l.tables + 2 * (size_t)S->loSize;
   l.withFactors = l.withLo + 16 * (size_t)S->nbrComplexFactors;
   l.factorsFit = l.free && S->d_rankLo16 && S->nbrOrbitals <= 32 && l.withFactors <= 160 * 1024;
+  l.withHi = l.withFactors + 4 * (size_t)S->hiSize;
+  l.hiFits = l.factorsFit && l.withHi <= 160 * 1024;
   return l;
 }
 
@@ -694,7 +714,7 @@ static int lattice_launch(dh_sector_set* S, int blockSize, const double* x, doub
   // the factors in LDS for a workgroup that fills its CU (16 wavefronts); smaller ones would leave it empty
   const bool facLds = l.factorsFit && blockSize == 1024;
   const bool loLds = S->d_rankLo16 && l.withLo <= 79 * 1024;  // two workgroups' tables in a CU's 160 KiB
-  const size_t lds = facLds ? l.withFactors : loLds ? l.withLo : l.tables;
+  const size_t lds = facLds ? (l.hiFits ? l.withHi : l.withFactors) : loLds ? l.withLo : l.tables;
   if (lds > 160 * 1024) return dh_fail(c, DH_E_RANGE, "staged tables exceed LDS");
   auto launch = [&](auto kern) -> int {
     if (lds > 64 * 1024)
@@ -707,7 +727,9 @@ static int lattice_launch(dh_sector_set* S, int blockSize, const double* x, doub
   };
   if (!l.free)
     return loLds ? launch(lattice_hv_kernel<K, LPR, true, 0, false>) : launch(lattice_hv_kernel<K, LPR, false, 0, false>);
-  if (facLds) return launch(lattice_hv_kernel<K, LPR, true, 32, true>);
+  if (facLds)
+    return l.hiFits ? launch(lattice_hv_kernel<K, LPR, true, 32, true, true>)
+                    : launch(lattice_hv_kernel<K, LPR, true, 32, true>);
   if (S->nbrOrbitals <= 32)
     return loLds ? launch(lattice_hv_kernel<K, LPR, true, 32, false>)
                  : launch(lattice_hv_kernel<K, LPR, false, 32, false>);
@@ -718,9 +740,9 @@ static int lattice_launch(dh_sector_set* S, int blockSize, const double* x, doub
 // Lanes per row and workgroup size by rows per CU and k, times in us on MI355X.  Few rows: lanes for
 // wavefronts (8008 rows: 21.0 with 4 x 256, 25.5 with 1 x 256; k = 4: 24.7 with 8 x 256, 40.8).  Up to
 // 512 rows a CU 2 x 512 (53 k rows: 27.0 against 34.9).  Above, where the factors fit LDS, 1 x 1024
-// with them there (177 k rows 55.9 against 63.6 at 1 x 256 and 61.4 at 2 x 512; 30 M rows 23.5 ms
+// with them there (177 k rows 50.9 against 63.3 at 1 x 256 and 60.9 at 2 x 512; 30 M rows 23.5 ms
 // against 31.1 and 29.7); for k > 2 the rows' own gathers weigh more and the line is at 2048 rows a CU
-// (177 k rows, k = 4: 145 at 1 x 256, 167 at 1 x 1024; 735 k rows: 986 against 670).  Where they don't
+// (177 k rows, k = 8: 355 at 1 x 256, 392 and more at 1 x 1024; 735 k rows, k = 4: 986 against 639).  Where they don't
 // fit, two lanes (1.9 M rows on 36 sites: 1698 at 2 x 512 against 1882; k = 4: 3509 at 2 x 256, 3856).
 static void lattice_shape(const dh_sector_set* S, int k, int* lpr, int* bs) {
   *lpr = S->lanesPerRow;

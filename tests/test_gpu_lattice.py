@@ -140,10 +140,11 @@ def test_momentum_element_counts_match_oracle_rows(arch):
 
 
 # 32 bits a word up to 32 orbitals, 64 above; the factors in LDS for 1024 threads where they fit
-# (30 orbitals, not 32); one row of momenta; no launch chosen (lpr 0)
+# (30 orbitals, not 32), the high rank table too up to 27; one row of momenta; no launch chosen (lpr 0)
 @pytest.mark.parametrize("n,nx,ny,lpr,block", [(3, 6, 5, 1, 1024), (3, 6, 5, 4, 1024), (4, 5, 3, 2, 1024),
                                                (3, 8, 4, 1, 1024), (3, 1, 32, 1, 256), (3, 11, 3, 2, 256),
-                                               (2, 8, 5, 8, 64), (2, 1, 37, 1, 256), (4, 5, 4, 0, 0)])
+                                               (2, 8, 5, 8, 64), (2, 1, 37, 1, 256), (4, 5, 4, 0, 0),
+                                               (3, 9, 3, 1, 1024), (3, 7, 4, 2, 1024)])
 @pytest.mark.parametrize("k", [1, 2, 8])
 def test_momentum_rows_at_word_and_table_limits(arch, n, nx, ny, lpr, block, k):
     sectors = [(0, 0), (nx - 1, 1), (nx // 2, ny - 1)]
