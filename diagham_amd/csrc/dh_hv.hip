@@ -644,8 +644,9 @@ template <int K>
 static int spin_dispatch(dh_hamiltonian* h, const double* x, double* y, int add, int64_t first, int64_t count) {
   if (h->indexMode == DH_INDEX_BSEARCH) return spin_bsearch_launch<K>(h, x, y, add, first, count);
   if (h->basis->dim >= (1ll << 31)) return dh_fail(h->ctx, DH_E_RANGE, "spin sector of 2^31 states or more");
-  if (dh_spin_tiles(h, K)) return dh_spin_tile_hv(h, spin_uniform(h), x, y, K, add, first, count);
-  if (spin_uniform(h)) return spin_rank_launch<K, true>(h, x, y, add, first, count);
+  const bool uniform = spin_uniform(h);
+  if (dh_spin_tiles(h, uniform, K)) return dh_spin_tile_hv(h, uniform, x, y, K, add, first, count);
+  if (uniform) return spin_rank_launch<K, true>(h, x, y, add, first, count);
   return spin_rank_launch<K, false>(h, x, y, add, first, count);
 }
 

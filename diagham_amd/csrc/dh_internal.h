@@ -224,7 +224,7 @@ struct dh_sector_set {
 // work descriptor of the active sectors (dh_multisector.hip)
 // tiled spin-1/2 product (dh_spin_tile.hip): its tables, whether it takes blocks of k, the product
 int dh_spin_tile_tables(dh_basis* b);
-bool dh_spin_tiles(const dh_hamiltonian* h, int k);
+bool dh_spin_tiles(const dh_hamiltonian* h, bool uniform, int k);
 int dh_spin_tile_hv(dh_hamiltonian* h, bool uniform, const double* x, double* y, int k, int add, int64_t first,
                     int64_t count);
 

@@ -390,15 +390,15 @@ static int spin_tile_sites(const dh_hamiltonian* h, int k) {
   }
 }
 
-// Enough tiles to fill the CUs twice, and half full ones on average: a tile costs 3.7 ns however few rows it
+// Enough tiles to fill the CUs twice (once with equal couplings, one vector), and half full ones on average: a tile costs 3.7 ns however few rows it
 // has (24 sites: Sz = 2, 0.52 full, 24.4 us against 35.8 by rows, k = 4 70.7 against 71.5; Sz = 4, 0.19
 // full, 19.7 against 20.4, k = 4 41 against 34; 28 sites, Sz = 4, 0.23 full, 205 against 195).  20 sites, 256 tiles of one vector: 6.4 and 9.3
 // us (equal and different couplings) against 6.9 by rows; 22 sites 9.7 and 12.1 against 18.8 and 17.3; two
 // vectors, 512 tiles, 14.9 against 20.4.
-bool dh_spin_tiles(const dh_hamiltonian* h, int k) {
+bool dh_spin_tiles(const dh_hamiltonian* h, bool uniform, int k) {
   const dh_basis* b = h->basis;
   const int lo = spin_tile_sites(h, k);
-  if (!b->d_spinTile || b->chainLength < lo + 9) return false;
+  if (!b->d_spinTile || b->chainLength < lo + (k == 1 && uniform ? 8 : 9)) return false;
   return 2 * (b->dim >> (b->chainLength - lo)) >= binom_c(lo, lo / 2);
 }
 

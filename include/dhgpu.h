@@ -151,7 +151,8 @@ int64_t dh_hamiltonian_dimension(const dh_hamiltonian* ham);
  * rows per wavefront; spin chains: 1); block_size a multiple of 64 up to 1024; index_mode
  * DH_INDEX_*; lds_tables != 0 stages the index tables in LDS when they fit.  Until it is called, a
  * sphere Hamiltonian picks its shape per product from k and its rows per CU: more lanes per row in
- * small workgroups on small spaces, 1024-thread workgroups on large ones. */
+ * small workgroups on small spaces, 1024-thread workgroups on large ones.  The tiled rank products of
+ * spin chains (long chains in well filled sectors) have a shape of their own. */
 int dh_hamiltonian_set_launch(dh_hamiltonian* ham, int lanes_per_row, int block_size, int index_mode, int lds_tables);
 
 /* ---------------------------------------------------------------- products
