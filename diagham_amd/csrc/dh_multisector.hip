@@ -515,7 +515,8 @@ static int sectors_hv_launch(dh_sector_set* S, int blockSize, bool freePairs, co
 // 1 x 256, 40 with 1 x 512 and 1 x 1024; k = 4: 55 with 2 x 256, 60 with 1 x 512, 71 by ranges; k = 8: 99, 125
 // by ranges; k = 16: 285 with 4 x 256, 375 with 2 x 512 by ranges).  Above, the tables in LDS bound the
 // wavefronts of a CU: 1024 threads (1.0 M rows: 188, 232 at 256; 17.6 M rows with 29 orbitals: 5.4 ms, 8.4 at
-// 512, 14.0 at 256), for k = 4 512 when three workgroups fit (1.0 M rows, 25 orbitals: 314, 336 at 1024, 425 by
+// 512, 14.0 at 256), 512 once x outgrows the 256 MB behind the L2s and the gathers go to HBM (278 M rows: 191
+// ms, 211 at 1024), for k = 4 512 when three workgroups fit (1.0 M rows, 25 orbitals: 314, 336 at 1024, 425 by
 // ranges).  k = 8: two lanes, 1024 threads where one workgroup's tables fill a CU (6.7 M rows: 6.0 ms, 7.0 with
 // 2 x 512), 512 where more fit (1.0 M rows: 676, 725 at 1024), one lane with the high table in L2 (17.6 M rows
 // 22.3 ms, 23.7 with two).  k = 16: two lanes, 512, and by ranges (2139, 2242 with the masks).
@@ -543,7 +544,7 @@ static void sectors_shape(const dh_sector_set* S, int k, int* lpr, int* bs, bool
     const bool three = 3 * sectors_lds(S, S->nbrSectors, 512, &tables) <= 160 * 1024;
     const bool oneFills = sectors_lds(S, S->nbrSectors, 1024, &tables) > 79 * 1024 && tables == 2;
     if (k <= 2)
-      set(1, 1024);
+      set(1, S->totalDim * k <= (int64_t)1 << 25 ? 1024 : 512);
     else if (k == 4)
       set(1, three && !oneFills ? 512 : 1024);
     else
