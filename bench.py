@@ -79,7 +79,7 @@ def load_traffic(name):
 
 def spin_hv_bench(capi, arch, stream, L, steps, warmup, k=1, index_mode=None):
     p = capi.Problem.spin_chain(arch, L, 0, 1.0, 1.0, True)
-    # 1024-thread workgroups: the fastest measured shape
+    # the tiled rank product has a shape of its own; 1024-thread workgroups are the fastest of the binary search
     p.set_launch(1, 1024, capi.INDEX_RANK if index_mode is None else index_mode, 1)
     nnz = p.count_elements()
     x = capi.DeviceBuffer(arch, p.dim * k)
@@ -235,9 +235,6 @@ def batched_hv_roofline(capi, arch, stream, n=12, lz=33, k=8, reps=3):
     pp = capi.coulomb_pseudopotentials(lz, True)
     lzs = capi.sphere_sectors(n, lz)
     S = capi.SphereSectorSet(arch, n, lz, lzs, pp)
-    # two lanes per row, 1024-thread workgroups: the sector solver's own shape for k >= 4, the fastest
-    # of the committed sweep (profiles/launch_shape_sweeps.md)
-    S.set_launch(2, 1024)
     nnz = int(S.count_elements().sum())
     x = capi.DeviceBuffer(arch, S.total * k)
     y = capi.DeviceBuffer(arch, S.total * k)
@@ -257,9 +254,8 @@ def batched_hv_roofline(capi, arch, stream, n=12, lz=33, k=8, reps=3):
     achieved = alg / (ms * 1e-3) / 1e9
     traffic = load_traffic("traffic_sectors_hv_n%d_2s%d_k%d.json" % (n, lz, k))
     return {"workload": "fermions_sphere_n%d_2s%d_all_Lz_ge_0_sectors_one_product_k%d" % (n, lz, k),
-            "kernel": "sectors_hv_kernel<%d, 2, true, false, false>" % k, "sectors": len(lzs), "rows": rows,
-            "launch": {"lanes_per_row": 2, "block_size": 1024, "row_routine": "range", "low_rank_table": "LDS, 16-bit",
-                       "chosen_by": "profiles/launch_shape_sweeps.md"},
+            "kernel": "sectors_hv_kernel<%d>" % k, "sectors": len(lzs), "rows": rows,
+            "launch": {"chosen_by": "the set, from its rows per CU and k"},
             "matrix_elements": nnz, "ms": ms, "element_vector_products_per_s": nnz * k / (ms * 1e-3),
             "algorithmic_bytes": alg, "achieved_GBps": achieved, "frac_of_peak": achieved / (HBM_PEAK / 1e9),
             "traffic": traffic and traffic["bytes_per_launch"],
@@ -370,7 +366,8 @@ def kernel_only(capi, arch, stream, name, steps, warmup):
     elif name.startswith("sectors_n12_2s33"):
         S = capi.SphereSectorSet(arch, 12, 33, capi.sphere_sectors(12, 33), capi.coulomb_pseudopotentials(33, True))
         cleanup.append(S.close)
-        S.set_launch(lpr or 2, bs or 1024) if k >= 4 else S.set_launch(lpr or 1, bs or 1024)
+        if lpr or bs:  # otherwise the set's own choice per k
+            S.set_launch(lpr or 1, bs or 1024)
         if free or rng:
             S.set_row_mode(capi.INDEX_RANK_FREE if free else capi.INDEX_RANK_RANGE)
         rows, nnz = S.total, int(S.count_elements().sum())
@@ -380,7 +377,8 @@ def kernel_only(capi, arch, stream, name, steps, warmup):
         from_lattice = capi.lattice_set(arch, 10, 6, 5, [x for x in range(6) for y in range(5)],
                                         [y for x in range(6) for y in range(5)])
         cleanup.append(from_lattice.close)
-        from_lattice.set_launch(lpr or (2 if k <= 2 else 1), bs or (512 if k <= 2 else 256))
+        if lpr or bs:
+            from_lattice.set_launch(lpr or 1, bs or 1024)
         if free or rng:
             arch.check(capi.gpu().dh_sector_set_row_mode(from_lattice.h, capi.INDEX_RANK_FREE if free
                                                          else capi.INDEX_RANK_RANGE), "row mode")
@@ -599,9 +597,9 @@ def main():
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                      "frac": achieved / (HBM_PEAK / 1e9),
                      "traffic": (traffic or {}).get("bytes_per_launch"),
-                     "kernel": "spin_rank_kernel<1, UNIFORM>", "algorithmic_bytes_per_launch": alg_bytes},
+                     "kernel": "spin_tile_kernel<1, 14, UNIFORM>", "algorithmic_bytes_per_launch": alg_bytes},
         # the algorithmic model reads x once per matrix element; L2 and MALL serve repeated reads, so
-        # the measured HBM bytes (rocprofv3 FETCH_SIZE + WRITE_SIZE) are fewer: their rate is the
+        # the measured HBM bytes (rocprofv3 read requests by size + WRITE_SIZE) are fewer: their rate is the
         # device's real HBM load, beside `achieved`
         "measured_traffic": traffic and {"bytes_per_launch": traffic["bytes_per_launch"],
                                          "GBps": traffic["bytes_per_launch"] / (ms * 1e-3) / 1e9,
@@ -609,15 +607,14 @@ def main():
                                          "counted_at_block_size": traffic.get("block_size")},
         "copy_calibration": calib,
         # three readings of the same kernel time: the algorithmic model above (x read once per
-        # matrix element, which the caches partly serve), the compulsory bytes (every 32-bit state
-        # word, x and y once each: what no implementation can avoid) and the HBM bytes the counters
-        # measured (rocprofv3 FETCH_SIZE + WRITE_SIZE)
+        # matrix element, which the caches partly serve), the compulsory bytes (x and y once each: what
+        # no implementation can avoid) and the HBM bytes the counters measured
         "roofline_readings": {
             "algorithmic_frac": achieved / (HBM_PEAK / 1e9),
-            "compulsory_bytes_per_launch": dim * (4 + 8 + 8),
-            "compulsory_frac": dim * (4 + 8 + 8) / (ms * 1e-3) / HBM_PEAK,
+            "compulsory_bytes_per_launch": dim * (8 + 8),
+            "compulsory_frac": dim * (8 + 8) / (ms * 1e-3) / HBM_PEAK,
             "counter_frac": traffic and traffic["bytes_per_launch"] / (ms * 1e-3) / HBM_PEAK,
-            "counter_over_compulsory": traffic and traffic["bytes_per_launch"] / (dim * (4 + 8 + 8)),
+            "counter_over_compulsory": traffic and traffic["bytes_per_launch"] / (dim * (8 + 8)),
         },
     }
     progress("headline product: %.3f ms" % ms)
