@@ -277,12 +277,15 @@ extern "C" int dh_spin_chain_create(dh_context* c, dh_basis** out, int L, int sz
   std::vector<uint32_t> binom(33 * 33, 0);
   for (int n = 0; n <= 32; ++n)
     for (int k = 0; k <= 32; ++k) binom[n * 33 + k] = (uint32_t)std::min<uint64_t>(dh_binom_host(n, k), 0xffffffffu);
+  const bool tiles = L >= 20;  // chains that the tiled product may take
+  const size_t wordBytes = (sizeof(uint32_t) * dim + 255) & ~size_t(255);
   int rc;
   if ((rc = upload(c, (void**)&b->d_binom, binom.data(), sizeof(uint32_t) * binom.size())) ||
-      (rc = dh_alloc(c, (void**)&b->d_words, sizeof(uint32_t) * dim))) {
+      (rc = dh_alloc(c, (void**)&b->d_words, wordBytes + (tiles ? dh_spin_tile_bytes() : 0)))) {
     dh_basis_destroy(b);
     return rc;
   }
+  if (tiles) b->d_spinTile = b->d_words + wordBytes / sizeof(uint32_t);
   hipLaunchKernelGGL(spin_unrank_kernel, dim3((unsigned)((dim + 255) / 256)), dim3(256), 0, c->stream, b->d_words,
                      dim, L, nbrUp, b->d_binom);
   b->lutBits = std::min(L, 14);
@@ -293,7 +296,7 @@ extern "C" int dh_spin_chain_create(dh_context* c, dh_basis** out, int L, int sz
   }
   hipLaunchKernelGGL(spin_lut_kernel, dim3((unsigned)(((1 << b->lutBits) + 1 + 255) / 256)), dim3(256), 0,
                      c->stream, b->d_words, dim, L, b->lutShift, b->lutBits, b->d_lut);
-  if (L >= 20 && (rc = dh_spin_tile_tables(b))) {
+  if (tiles && (rc = dh_spin_tile_tables(b))) {
     dh_basis_destroy(b);
     return rc;
   }
@@ -313,7 +316,6 @@ extern "C" int dh_basis_destroy(dh_basis* b) {
   hipStreamSynchronize(c->stream);
   if (b->d_states) hipFree(b->d_states);
   if (b->d_words) hipFree(b->d_words);
-  if (b->d_spinTile) hipFree(b->d_spinTile);
   if (b->d_lut) hipFree(b->d_lut);
   if (b->d_rankLo) hipFree(b->d_rankLo);
   if (b->d_rankHi) hipFree(b->d_rankHi);

@@ -108,7 +108,7 @@ struct dh_basis {
   uint16_t* d_rankLo16 = nullptr;
   // binomial table C[n][k], n,k <= 32 (spin rank)
   uint32_t* d_binom = nullptr;
-  uint32_t* d_spinTile = nullptr;  // pattern tables of the tiled spin product (dh_spin_tile_tables)
+  uint32_t* d_spinTile = nullptr;  // pattern tables of the tiled spin product, behind d_words (dh_spin_tile_tables)
 };
 
 enum dh_ham_kind { DH_HAM_SPHERE = 1, DH_HAM_SPIN = 2, DH_HAM_SPHERE_NBODY = 3 };
@@ -223,6 +223,7 @@ struct dh_sector_set {
 
 // work descriptor of the active sectors (dh_multisector.hip)
 // tiled spin-1/2 product (dh_spin_tile.hip): its tables, whether it takes blocks of k, the product
+size_t dh_spin_tile_bytes();
 int dh_spin_tile_tables(dh_basis* b);
 bool dh_spin_tiles(const dh_hamiltonian* h, bool uniform, int k);
 int dh_spin_tile_hv(dh_hamiltonian* h, bool uniform, const double* x, double* y, int k, int add, int64_t first,

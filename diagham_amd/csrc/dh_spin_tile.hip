@@ -368,10 +368,10 @@ int spin_tile_launch(dh_hamiltonian* h, bool uniform, const double* x, double* y
 
 }  // namespace
 
+size_t dh_spin_tile_bytes() { return sizeof(uint32_t) * (tile_offset(kLoMax + 1) + kZeroWords); }
+
 int dh_spin_tile_tables(dh_basis* b) {
   dh_context* c = b->ctx;
-  int rc = dh_alloc(c, (void**)&b->d_spinTile, sizeof(uint32_t) * (tile_offset(kLoMax + 1) + kZeroWords));
-  if (rc) return rc;
   hipLaunchKernelGGL(spin_tile_table_kernel, dim3(kZeroWords / 256, kLoMax - kLoMin + 2), dim3(256), 0, c->stream,
                      b->d_spinTile, b->d_binom);
   DH_HIP(c, hipGetLastError());
