@@ -441,8 +441,8 @@ __global__ void __launch_bounds__(kAdjointThreads) sphere_adjoint_kernel(int nbr
             const int i = __builtin_ctz(pm);
             pm &= pm - 1;
             const U w = t | (U(1) << (m3lo + i)) | (U(1) << (m4hi - i));
-            // clamped so that a target outside the sector can never address outside the vectors
-            idx[q] = min(dh_word(hi, (uint32_t)(w >> rankBits)) - dh_word(lo, (uint32_t)(w & loMask)), last);
+            constexpr bool FAR = dh_far_tables<U, false>;
+            idx[q] = dh_rank_of<FAR>(w, dh_entry<FAR>(lo, (uint32_t)(w & loMask)), hi, rankBits, last);
             pos[q] = i;
           }
         }

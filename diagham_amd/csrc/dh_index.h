@@ -23,9 +23,27 @@ __device__ __forceinline__ int64_t dh_find_bsearch(uint64_t target, const int* _
   return lo;  // in [lut[key+1], lut[key]) for every target of the sector
 }
 
-// Entry i of a table of less than 2^30 words, by a 32-bit byte offset (one address instruction)
-__device__ __forceinline__ uint32_t dh_word(const uint32_t* __restrict__ table, uint32_t i) {
+// Entry i of a rank table.  FAR: any i; otherwise the table has at most 2^30 words and its byte offset is
+// 32 bits long (one address instruction instead of two).
+template <bool FAR>
+__host__ __device__ __forceinline__ uint32_t dh_entry(const uint32_t* __restrict__ table, uint32_t i) {
+  if constexpr (FAR) return table[i];
   return *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(table) + (i << 2));
+}
+
+// Which rank tables are FAR.  States on words U of 32 bits have at most 32 orbitals, and a low table that is
+// short enough for LDS (2^15 entries) comes with a high one of 2^20 at most (dh_rank_split).  The others
+// reach 2^31 words: 62 orbitals (the high one; the low one from 61 on).
+template <typename U, bool LO_IN_LDS>
+constexpr bool dh_far_tables = sizeof(U) == 8 && !LO_IN_LDS;
+
+// Rank of state t in 32 bits from the entry `lo` of its low orbitals and the high table, clamped so that a
+// target outside the sector (of last + 1 states) can never address outside the vectors.
+template <bool FAR, typename U>
+__host__ __device__ __forceinline__ uint32_t dh_rank_of(U t, uint32_t lo, const uint32_t* __restrict__ hi, int bits,
+                                                        uint32_t last) {
+  const uint32_t r = dh_entry<FAR>(hi, (uint32_t)(t >> bits)) - lo;
+  return r < last ? r : last;
 }
 
 // Combinatorial rank of a fermion state in the descending basis of its sector (the low table in 32

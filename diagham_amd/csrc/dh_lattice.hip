@@ -550,9 +550,8 @@ __global__ void __launch_bounds__(1024) lattice_hv_kernel(LatticeArgs a, const d
       const LatticeTables T{sFacOff, sMask, sDiag, sInfo, sPairOff, sShift, sPP};
       const uint32_t last = (uint32_t)dim - 1u, mask = (uint32_t)a.loSize - 1u;
       const int bits = a.rankBits;
-      // clamped so that a target outside the sector can never address outside the vectors
       auto find = [&](U t) -> uint32_t {
-        return min(dh_word(hi, (uint32_t)(t >> bits)) - lo[(uint32_t)t & mask], last);
+        return dh_rank_of<dh_far_tables<U, LO_LDS>>(t, lo[(uint32_t)t & mask], hi, bits, last);
       };
       const double2* fac;
       if constexpr (FAC_LDS)
