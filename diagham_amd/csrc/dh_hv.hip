@@ -571,10 +571,6 @@ static int sphere_dispatch_lpr(dh_hamiltonian* h, const double* x, double* y, in
       set(2, 1024);
     }
   }
-  // k = 2 with one lane per row faulted the GPU twice on N=5 2S=33 (free-pair rows, with the low
-  // rank table in LDS and in global memory) with no cause found in the code; k = 2 runs with two
-  // lanes per row, as tested, until one is
-  if (K == 2 && lpr == 1) lpr = 2;
   switch (lpr) {
     case 1: return sphere_dispatch_mode<K, 1>(h, bs, freePairs, x, y, add, first, count);
     case 2: return sphere_dispatch_mode<K, 2>(h, bs, freePairs, x, y, add, first, count);

@@ -1,0 +1,46 @@
+"""Products of sector sets in the launch shapes that the sets choose by themselves and in the forms of the row
+routine that such a choice reaches, every column of a block against the oracle."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+from test_gpu_sectors import SectorSet, coulomb
+
+pytestmark = pytest.mark.gpu
+
+
+def sphere_set_matches(S, n, lz_max, sectors, V, k, rows=None):
+    """H of a set against the oracle in every column; rows: only that many rows of each sector, spread over it"""
+    fac = O.Factors(lz_max, V)
+    X = np.random.default_rng(lz_max + k).standard_normal((S.total, k))
+    Y = S.hv(X.reshape(-1), k).reshape(S.total, k)
+    for i, lz in enumerate(sectors):
+        ref = O.FermionSphere(n, lz, lz_max)
+        a, b = S.off[i], S.off[i + 1]
+        assert b - a == ref.dim
+        x = np.ascontiguousarray(X[a:b])
+        if rows is None or ref.dim <= rows:
+            y = np.stack([O.fs_hv(ref, fac, np.ascontiguousarray(x[:, v])) for v in range(k)], axis=1)
+            got = Y[a:b]
+        else:
+            at = np.unique(np.linspace(0, ref.dim - 1, rows).astype(int))
+            y = np.zeros((at.size, k))
+            for j, r in enumerate(at):
+                t, c = O.fs_row_elements(ref, fac, int(r))
+                y[j] = c @ x[t]
+            got = Y[a:b][at]
+        for v in range(k):
+            assert np.linalg.norm(got[:, v] - y[:, v]) <= 1e-12 * max(np.linalg.norm(y[:, v]), 1e-300), (lz, k, v)
+
+
+# one lane per row on 64-bit words: the low rank table in LDS (34 orbitals) and both in global memory (36)
+@pytest.mark.parametrize("n,lz_max,sectors", [(4, 33, [0, 2, 12, 90]), (4, 35, [0, 2, 10, 60])])
+@pytest.mark.parametrize("k,row_mode", [(1, 1), (2, 1), (2, 3), (2, 4), (4, 3), (8, 1), (8, 3)])
+@pytest.mark.parametrize("block", [256, 1024])
+def test_sector_rows_on_one_lane_of_64_bit_words(arch, n, lz_max, sectors, k, row_mode, block):
+    V = coulomb(lz_max)
+    S = SectorSet(arch, n, lz_max, sectors, V)
+    assert S.capi.gpu().dh_sector_set_row_mode(S.h, row_mode) == 0
+    assert S.capi.gpu().dh_sector_set_launch(S.h, 1, block) == 0
+    sphere_set_matches(S, n, lz_max, sectors, V, k)
+    S.close()

@@ -384,10 +384,6 @@ def test_hv_parity_at_the_14_bit_rank_split(arch, n, total_lz, lz_max, k, launch
     """29 to 34 orbitals: the rank tables split at 14 bits, the 16-bit low table staged in LDS and
     the high table (2^15 to 2^20 entries) read from global memory; the automatic launch and explicit
     shapes of each row routine, 32-bit (32 orbitals) and 64-bit state words."""
-    if launch in ((1, 1024, 1), (1, 512, 3)) and k == 2 and (n, total_lz, lz_max) == (5, 1, 33):
-        pytest.skip("faulted the GPU (k = 2, one lane per row, free-pair rows, 34 orbitals; with the low "
-                    "rank table in LDS and in global memory) with no cause found; the dispatch runs k = 2 "
-                    "with two lanes per row instead until one is")
     from diagham_amd import capi
     p = capi.Problem.sphere(arch, n, total_lz, lz_max, coulomb(lz_max))
     ref_space = O.FermionSphere(n, total_lz, lz_max)
