@@ -160,14 +160,15 @@ __global__ void __launch_bounds__(1024) sphere_hv_kernel(SphereArgs a, const dou
     double acc[K];
 #pragma unroll
     for (int v = 0; v < K; ++v) acc[v] = 0.0;
+    dh_diagonal diag;
     if constexpr (WORDS == 1 && BASE != MODE_BSEARCH) {
       const uint32_t last = (uint32_t)a.dim - 1u, mask = (1u << a.rankBits) - 1u;
       const int bits = a.rankBits;
       auto find = [&](uint32_t t) -> uint32_t { return dh_rank_of<false>(t, loAt(t & mask), sHi, bits, last); };
       if constexpr (ROW == ROW_X4)
-        dh_sphere_row_x4<K, LPR, TRI>((uint32_t)s, a.nbrOrbitals, sF, sBase, lane, find, x, (uint32_t)row, acc);
+        diag = dh_sphere_row_x4<K, LPR, TRI>((uint32_t)s, a.nbrOrbitals, sF, sBase, lane, find, x, acc);
       else
-        dh_sphere_row<K, LPR, ROW == ROW_FREE, TRI>((uint32_t)s, a.nbrOrbitals, sF, sBase, lane, find, x, (uint32_t)row, acc);
+        diag = dh_sphere_row<K, LPR, ROW == ROW_FREE, TRI>((uint32_t)s, a.nbrOrbitals, sF, sBase, lane, find, x, acc);
     } else if constexpr (WORDS == 2 && BASE != MODE_BSEARCH) {
       // rankBits = ceil(orbitals / 2) <= 32, so t >> bits fits 32 bits
       const uint32_t last = (uint32_t)a.dim - 1u;
@@ -177,15 +178,15 @@ __global__ void __launch_bounds__(1024) sphere_hv_kernel(SphereArgs a, const dou
         return dh_rank_of<dh_far_tables<uint64_t, BASE != MODE_RANK_GLOBAL>>(t, loAt((uint32_t)t & mask), sHi, bits, last);
       };
       if constexpr (ROW == ROW_X4)
-        dh_sphere_row_x4<K, LPR, TRI>(s, a.nbrOrbitals, sF, sBase, lane, find, x, (uint32_t)row, acc);
+        diag = dh_sphere_row_x4<K, LPR, TRI>(s, a.nbrOrbitals, sF, sBase, lane, find, x, acc);
       else
-        dh_sphere_row<K, LPR, ROW == ROW_FREE, TRI>(s, a.nbrOrbitals, sF, sBase, lane, find, x, (uint32_t)row, acc);
+        diag = dh_sphere_row<K, LPR, ROW == ROW_FREE, TRI>(s, a.nbrOrbitals, sF, sBase, lane, find, x, acc);
     } else {
       auto find = [&](uint64_t t) -> int64_t { return sphere_find<BASE>(a, t, sLut, sLo, sHi, sLo16); };
       if constexpr (ROW == ROW_X4)
-        dh_sphere_row_x4<K, LPR, TRI>(s, a.nbrOrbitals, sF, sBase, lane, find, x, row, acc);
+        diag = dh_sphere_row_x4<K, LPR, TRI>(s, a.nbrOrbitals, sF, sBase, lane, find, x, acc);
       else
-        dh_sphere_row<K, LPR, ROW == ROW_FREE, TRI>(s, a.nbrOrbitals, sF, sBase, lane, find, x, row, acc);
+        diag = dh_sphere_row<K, LPR, ROW == ROW_FREE, TRI>(s, a.nbrOrbitals, sF, sBase, lane, find, x, acc);
     }
     if constexpr (LPR > 1) {
 #pragma unroll
@@ -196,7 +197,7 @@ __global__ void __launch_bounds__(1024) sphere_hv_kernel(SphereArgs a, const dou
       const double* xr = x + row * K;
       double* yr = y + row * K;
 #pragma unroll
-      for (int v = 0; v < K; ++v) yr[v] = (add ? yr[v] : 0.0) + acc[v] + a.shift * xr[v];
+      for (int v = 0; v < K; ++v) yr[v] = (add ? yr[v] : 0.0) + diag.term(xr[v], acc[v]) + a.shift * xr[v];
     }
   }
 }

@@ -388,12 +388,12 @@ __global__ void __launch_bounds__(1024) sectors_hv_kernel(SectorsArgs a, const d
     double acc[K];
 #pragma unroll
     for (int v = 0; v < K; ++v) acc[v] = 0.0;
+    dh_diagonal diag;
     if constexpr (S32) {
       const uint32_t last = (uint32_t)dim - 1u, mask = (1u << a.rankBits) - 1u;
       const int bits = a.rankBits;
       auto find = [&](uint32_t t) -> uint32_t { return dh_rank_of<false>(t, loAt(t & mask), hi, bits, last); };
-      dh_sphere_row<K, LPR, FREE, TRI>((uint32_t)s, a.nbrOrbitals, sF, sBase, lane, find, x + off * K,
-                                       (uint32_t)(g - off), acc);
+      diag = dh_sphere_row<K, LPR, FREE, TRI>((uint32_t)s, a.nbrOrbitals, sF, sBase, lane, find, x + off * K, acc);
     } else {
       // rankBits = ceil(orbitals / 2) <= 32, so t >> bits fits 32 bits
       const uint32_t last = (uint32_t)dim - 1u;
@@ -402,8 +402,7 @@ __global__ void __launch_bounds__(1024) sectors_hv_kernel(SectorsArgs a, const d
       auto find = [&](uint64_t t) -> uint32_t {
         return dh_rank_of<dh_far_tables<uint64_t, (TABLES > 0)>>(t, loAt((uint32_t)t & mask), hi, bits, last);
       };
-      dh_sphere_row<K, LPR, FREE, TRI>(s, a.nbrOrbitals, sF, sBase, lane, find, x + off * K,
-                                       (uint32_t)(g - off), acc);
+      diag = dh_sphere_row<K, LPR, FREE, TRI>(s, a.nbrOrbitals, sF, sBase, lane, find, x + off * K, acc);
     }
     if constexpr (LPR > 1) {
 #pragma unroll
@@ -414,7 +413,7 @@ __global__ void __launch_bounds__(1024) sectors_hv_kernel(SectorsArgs a, const d
       const double* xr = x + g * K;
       double* yr = y + g * K;
 #pragma unroll
-      for (int v = 0; v < K; ++v) yr[v] = (add ? yr[v] : 0.0) + acc[v] + a.shift * xr[v];
+      for (int v = 0; v < K; ++v) yr[v] = (add ? yr[v] : 0.0) + diag.term(xr[v], acc[v]) + a.shift * xr[v];
     }
   }
 }

@@ -92,9 +92,27 @@ __device__ __forceinline__ double dh_negate_by(double c, uint32_t signAtBit31) {
   return __hiloint2double(__double2hiint(c) ^ (int)(signAtBit31 & 0x80000000u), __double2loint(c));
 }
 
+// The diagonal coefficient of a row, -F(a, a) over its pairs a, in two doubles: each n1's pairs are subtracted
+// together, and what the subtraction rounds off is kept (Dekker's fast two-sum: exact while the sum is the
+// larger, which it is from the third n1 on for factors of one sign).  The caller adds the diagonal term last,
+// after the sums of the row's lanes have met: it is the largest by far, so a rounding after it costs the most.
+// Error against exactly summed elements, relative to the norm of the product: N=6 2S=15, k = 8, 1.26e-16 with
+// one double and the term on lane 0, 0.92 with the elements one by one, 0.59 so; N=8 2S=21 1.22, 1.13 and 0.59;
+// N=10 2S=27 1.09, 4.15 and 0.56.
+struct dh_diagonal {
+  double sum = 0.0, rest = 0.0;
+  __device__ __forceinline__ void subtract(double v) {
+    const double s = sum - v;
+    rest += (sum - s) - v;
+    sum = s;
+  }
+  // acc + this times x
+  __device__ __forceinline__ double term(double x, double acc) const { return fma(sum, x, fma(rest, x, acc)); }
+};
+
 // Two-body terms of row state s: for every occupied pair n1 > n2 (annihilated) and every other pair
 // m3 > m4 of the same orbital sum that is free in s (created), one gather; the diagonal terms are
-// summed into one coefficient of x[self].  FREE walks the set bits of the free mask; otherwise every
+// summed into one coefficient (returned, the same on every lane).  FREE walks the set bits of the free mask; otherwise every
 // position is tried against it (fewer registers).  Positions run from the highest down, and lane
 // `lane` of the row's LPR lanes takes every LPR-th (free) one.  Target indices come from
 // `find(target)`; x is indexed relative to `xbase`.
@@ -108,20 +126,21 @@ __device__ __forceinline__ double dh_negate_by(double c, uint32_t signAtBit31) {
 // are still added in their order, so FREE and the range form agree to the bit at one lane per row).
 // Wider K keep one gather in flight per term: their registers would lower the occupancy that hides
 // the latency there.
-template <int K, int LPR, bool FREE, bool TRI, typename U, typename Find, typename I>
-__device__ __forceinline__ void dh_sphere_row(U s, int nbrOrbitals, const double* __restrict__ sF,
-                                              const int* __restrict__ sBase, int lane, Find find,
-                                              const double* __restrict__ xbase, I self, double* acc) {
+template <int K, int LPR, bool FREE, bool TRI, typename U, typename Find>
+__device__ __forceinline__ dh_diagonal dh_sphere_row(U s, int nbrOrbitals, const double* __restrict__ sF,
+                                                     const int* __restrict__ sBase, int lane, Find find,
+                                                     const double* __restrict__ xbase, double* acc) {
   constexpr bool PIPE = K <= 2;
   double pend[K];
-  double pendCoef = 0.0, diag = 0.0;
+  double pendCoef = 0.0;
+  dh_diagonal diag;
 #pragma unroll
   for (int v = 0; v < K; ++v) pend[v] = 0.0;
   const dh_row_masks<U> masks(s, nbrOrbitals);
   for (U r1 = s; r1; r1 &= r1 - 1) {
     const int n1 = dh_ctz(r1);
     const double* diagRow = sF + __mul24(n1, n1 - 1) / 2;  // !TRI
-    double diag1 = 0.0;  // of this n1: two short sums round less than one long one
+    double diag1 = 0.0;  // of this n1
     for (U r2 = s & ((U(1) << n1) - U(1)); r2; r2 &= r2 - 1) {
       const int n2 = dh_ctz(r2);
       if (!TRI) diag1 += diagRow[n2];
@@ -168,13 +187,13 @@ __device__ __forceinline__ void dh_sphere_row(U s, int nbrOrbitals, const double
           if ((pm >> j) & 1u) term(31 - j, 1u << j, q << (31 - j));
       }
     }
-    diag -= diag1;
+    diag.subtract(diag1);
   }
   if constexpr (PIPE) {
 #pragma unroll
     for (int v = 0; v < K; ++v) acc[v] = fma(pendCoef, pend[v], acc[v]);
   }
-  if (lane == 0) dh_gather_fma<K>(acc, xbase, self, diag);
+  return diag;
 }
 
 // The same terms with the created-pair loop unrolled four-wide: a lane computes four targets
@@ -182,12 +201,12 @@ __device__ __forceinline__ void dh_sphere_row(U s, int nbrOrbitals, const double
 // coefficient), issues their index lookups together and then their four gathers, so four
 // dependent chains are in flight per lane.  `s` must be a state of the space (the padding
 // slots look it up).
-template <int K, int LPR, bool TRI, typename U, typename Find, typename I>
-__device__ __forceinline__ void dh_sphere_row_x4(U s, int nbrOrbitals, const double* __restrict__ sF,
-                                                 const int* __restrict__ sBase, int lane, Find find,
-                                                 const double* __restrict__ xbase, I self, double* acc) {
+template <int K, int LPR, bool TRI, typename U, typename Find>
+__device__ __forceinline__ dh_diagonal dh_sphere_row_x4(U s, int nbrOrbitals, const double* __restrict__ sF,
+                                                        const int* __restrict__ sBase, int lane, Find find,
+                                                        const double* __restrict__ xbase, double* acc) {
   const dh_row_masks<U> masks(s, nbrOrbitals);
-  double diag = 0.0;
+  dh_diagonal diag;
   for (U r1 = s; r1; r1 &= r1 - 1) {
     const int n1 = dh_ctz(r1);
     double diag1 = 0.0;
@@ -216,7 +235,7 @@ __device__ __forceinline__ void dh_sphere_row_x4(U s, int nbrOrbitals, const dou
         for (int u = 0; u < 4; ++u) dh_gather_fma<K>(acc, xbase, idx[u], coef[u]);
       }
     }
-    diag -= diag1;
+    diag.subtract(diag1);
   }
-  if (lane == 0) dh_gather_fma<K>(acc, xbase, self, diag);
+  return diag;
 }
