@@ -388,8 +388,9 @@ int dh_spin_tile_tables(dh_basis* b) {
   return DH_OK;
 }
 
-// Last sites per tile: about 30 KB of x, so that five tiles' workgroups share a CU's LDS; for one vector on
-// chains below 26 sites 12, for more and smaller tiles (24 sites 25.6 us, 27.5 with 14; 28 sites 501 and 454).
+// Last sites per tile.  About 30 KB of x, 31 to 35 KB of LDS with the distances, so that four (k = 16 and the
+// 512-thread workgroups, by their wavefronts as well) or five (k = 8) tiles share a CU; for one vector on chains
+// below 26 sites 12, for more and smaller tiles (24 sites 25.6 us, 27.5 with 14; 28 sites 501 and 454).
 static int spin_tile_sites(const dh_hamiltonian* h, int k) {
   switch (k) {
     case 1: return h->basis->chainLength >= 26 ? 14 : 12;
@@ -400,16 +401,27 @@ static int spin_tile_sites(const dh_hamiltonian* h, int k) {
   }
 }
 
-// Enough tiles to fill the CUs twice (once with equal couplings, one vector), and half full ones on average: a tile costs 3.7 ns however few rows it
-// has (24 sites: Sz = 2, 0.52 full, 24.4 us against 35.8 by rows, k = 4 70.7 against 71.5; Sz = 4, 0.19
-// full, 19.7 against 20.4, k = 4 41 against 34; 28 sites, Sz = 4, 0.23 full, 205 against 195).  20 sites, 256 tiles of one vector: 6.4 and 9.3
-// us (equal and different couplings) against 6.9 by rows; 22 sites 9.7 and 12.1 against 18.8 and 17.3; two
-// vectors, 512 tiles, 14.9 against 20.4.
+// Enough tiles to fill the CUs, and rows enough in them: a tile costs 3.7 ns however few rows it has.  Lines where
+// the time by rows and by tiles meet, with that of the row kernel first (us):
+// - one vector, equal couplings: from 256 tiles on a ring (20 sites 7.0 and 6.5), 512 on an open chain (20
+//   sites 6.0 and 6.3, 21 sites 8.2 and 7.0); different ones from 1024 (21 sites 9.1 and 10.1 open, 10.3 and
+//   10.2 on a ring; 22 sites 17.6 and 12.3).  Blocks of k: from 512 (21 sites, k = 4: 15.1 and 13.2).
+// - tiles half full on average (24 sites, Sz = 4, 0.52 full: 39.0 and 30.7, k = 4 71.8 and 71.0), 0.6 with
+//   different couplings on open chains of few tiles (22 sites, 0.53 full: 11.0 and 11.9, k = 4 18.3 and 20.2).
+// - two vectors, whose rows of 16 bytes gain least: 0.6 with equal couplings (24 sites, 0.56 full: 37.4 and
+//   39.3; 23 sites, 0.65 full: 26.9 and 22.7); with different ones on a ring 0.6 up to 1024 tiles (22 sites, 0.57
+//   full: 14.0 and 15.7; 23 sites, 0.65 full: 29.6 and 25.9) and 0.7 above (26 sites, 0.69 full: 202 and 206; 0.74
+//   full: 216 and 210), on an open chain 0.7 with 512 tiles (22 sites, 0.73 full: 17.9 and 16.9) and never with
+//   more (24 sites, 0.71 full: 43.0 and 45.9; 26 sites, 0.74 full: 201 and 203).
 bool dh_spin_tiles(const dh_hamiltonian* h, bool uniform, int k) {
   const dh_basis* b = h->basis;
-  const int lo = spin_tile_sites(h, k);
-  if (!b->d_spinTile || b->chainLength < lo + (k == 1 && uniform ? 8 : 9)) return false;
-  return 2 * (b->dim >> (b->chainLength - lo)) >= binom_c(lo, lo / 2);
+  const int lo = spin_tile_sites(h, k), split = b->chainLength - lo;
+  const bool ring = h->periodic != 0;
+  if (!b->d_spinTile || split < (k == 1 ? (uniform ? (ring ? 8 : 9) : 10) : 9)) return false;
+  if (k == 2 && !uniform && !ring && split > 9) return false;
+  int tenths = !uniform && !ring && split <= 10 ? 6 : 5;
+  if (k == 2) tenths = uniform || (ring && split <= 10) ? 6 : 7;
+  return 10 * (b->dim >> split) >= (int64_t)tenths * binom_c(lo, lo / 2);
 }
 
 int dh_spin_tile_hv(dh_hamiltonian* h, bool uniform, const double* x, double* y, int k, int add, int64_t first,
