@@ -534,10 +534,16 @@ static int sphere_dispatch_lpr(dh_hamiltonian* h, const double* x, double* y, in
   // their registers cost more than they save (7.5 against 6.4)
   bool freePairs = h->indexMode == DH_INDEX_RANK_FREE || (h->indexMode == DH_INDEX_RANK && K <= (h->autoLaunch ? 8 : 2));
   if (h->autoLaunch) {
-    // The fastest shapes measured on MI355X by rows per CU and k, times in us.  Few rows: eight lanes, whose
-    // rows finish together with the range loop (338 rows: 7.7, 9.2 with 2 x 256 and the masks; 13 k rows 18.9
-    // and 20.6; k = 8 15.9 and 17.7).  Then lanes for wavefronts in small workgroups (45 k rows: 26.2 with
-    // 2 x 512, 36.8 with 4 x 512; k = 4 37.0 with 2 x 512, 43.1 by ranges; k = 8 50.7 with 4 x 256; 71 k rows:
+    // The fastest shapes measured on MI355X by rows per CU, k and the bytes of the staged tables, times in us.
+    // Few rows: eight lanes, whose rows finish together with the range loop (338 rows: 7.4, 9.2 with 2 x 256 and
+    // the masks).  The time is that of the staging and of one row's lookups, so large tables are staged by more
+    // threads: 512 up to k = 4 (85 rows on 27 orbitals 8.2, 12.1 with 256; 4370 on 25 12.2, 14.5; but 338 on 16
+    // 7.5 and 8.0) and, for k = 8, on 25 to 34 orbitals (14 k rows 25.0, 29.0; on 22 orbitals 19.7 and 18.6).  From
+    // 64 rows a CU 1024 (17 k rows 16.3, 24.3 with 2 x 512 and the masks; k = 4 22.9, 34.6), with blocks of 8 and
+    // 16 four lanes and the masks (24 k rows, k = 8: 38.4, 42.9 with 4 x 256).  Then lanes for wavefronts in
+    // smaller workgroups (45 k rows: 26.2 with 2 x 512, 36.8 with 4 x 512; k = 4 37.0 with 2 x 512, 43.1 by
+    // ranges; k = 8 51.2 with 4 x 256, but where fewer than three workgroups of 256 fit a CU 2 x 512, 60 k
+    // rows on 32 orbitals 76, 98 at 4 x 256; 71 k rows:
     // 37.9 with 1 x 512, 53 with 1 x 1024; k = 4 54.9 with 2 x 1024).  Many rows: the tables in LDS leave two
     // workgroups a CU or one, so 1024 threads (1.4 M rows: 603, 645 at 512); with the high table in L2 (not
     // both in LDS) k = 4 and 8 run better on fewer wavefronts (1.4 M rows: 1377 with 1 x 512, 1436 at 1024, and
@@ -547,12 +553,16 @@ static int sphere_dispatch_lpr(dh_hamiltonian* h, const double* x, double* y, in
     // k <= 2, 1024 above.
     const int64_t perCU = h->basis->dim / h->ctx->nbrCU;
     const int tables = sphere_rank_tables(h, K, 1024);
+    const size_t staged = sphere_lds(h, tables, 0);
     auto set = [&](int l, int b) { lpr = l, bs = b; };
     if (perCU < 64) {
-      set(8, 256);
+      set(8, K <= 4 ? (staged > 16 * 1024 ? 512 : 256) : K == 8 && tables != MODE_RANK_GLOBAL && staged > 40 * 1024 ? 512 : 256);
       freePairs = false;
+    } else if (perCU < 128) {
+      K <= 4 ? set(8, 1024) : set(4, tables == MODE_RANK_GLOBAL ? 256 : 512);
+      freePairs = K > 4;
     } else if (perCU < 256) {
-      K <= 4 ? set(2, 512) : set(4, 256);
+      K <= 4 || staged > 50 * 1024 ? set(2, 512) : set(4, 256);
       freePairs = true;
     } else if (tables == MODE_RANK_GLOBAL) {
       set(2, K <= 2 ? 256 : 1024);

@@ -44,3 +44,26 @@ def test_sector_rows_on_one_lane_of_64_bit_words(arch, n, lz_max, sectors, k, ro
     assert S.capi.gpu().dh_sector_set_launch(S.h, 1, block) == 0
     sphere_set_matches(S, n, lz_max, sectors, V, k)
     S.close()
+
+
+# a space in every branch of the rule below 256 rows per CU: few rows with small and large tables, from 64 and from
+# 128 rows per CU, with the low rank table in LDS and in global memory
+@pytest.mark.parametrize("n,total_lz,lz_max", [(6, 0, 15), (3, 0, 26), (5, 0, 36), (6, 1, 31), (5, 0, 44), (7, 0, 30),
+                                               (6, 0, 40)])
+@pytest.mark.parametrize("k", [1, 4, 8, 16])
+def test_small_spaces_in_their_own_shape(arch, n, total_lz, lz_max, k):
+    from diagham_amd import capi
+    total_lz += (n * lz_max + total_lz) % 2
+    V = coulomb(lz_max)
+    p = capi.Problem.sphere(arch, n, total_lz, lz_max, V)
+    X = np.random.default_rng(n + k).standard_normal((p.dim, k))
+    Y = p.hv(X.reshape(-1), k).reshape(p.dim, k)
+    p.close()
+    space, fac = O.FermionSphere(n, total_lz, lz_max), O.Factors(lz_max, V)
+    at = np.unique(np.linspace(0, space.dim - 1, 500).astype(int))
+    y = np.zeros((at.size, k))
+    for j, r in enumerate(at):
+        t, c = O.fs_row_elements(space, fac, int(r))
+        y[j] = c @ X[t]
+    for v in range(k):
+        assert np.linalg.norm(Y[at][:, v] - y[:, v]) <= 1e-12 * np.linalg.norm(y[:, v]), v
