@@ -33,10 +33,23 @@ struct dh_row_factors {
   }
 };
 
-template <int K, typename I>
+// ALL: every load of the row is issued before the first multiply-add.  The compiler does that by itself up to 8
+// vectors; for 16 it may take two loads at a time, for a fifth wavefront per SIMD that the LDS does not allow (3.4 M
+// rows of 28 orbitals: 8.6 ms with the loads together, 10.0 in twos).
+template <int K, bool ALL = false, typename I>
 __device__ __forceinline__ void dh_gather_fma(double* acc, const double* __restrict__ x, I idx, double coef) {
   const double* xr = x + (size_t)idx * K;
-  if constexpr (K % 2 == 0) {
+  if constexpr (ALL) {
+    double2 p[K / 2];
+#pragma unroll
+    for (int v = 0; v < K / 2; ++v) p[v] = reinterpret_cast<const double2*>(xr)[v];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int v = 0; v < K / 2; ++v) {
+      acc[2 * v] += coef * p[v].x;
+      acc[2 * v + 1] += coef * p[v].y;
+    }
+  } else if constexpr (K % 2 == 0) {
 #pragma unroll
     for (int v = 0; v < K; v += 2) {
       double2 p = *reinterpret_cast<const double2*>(xr + v);
@@ -167,7 +180,7 @@ __device__ __forceinline__ dh_diagonal dh_sphere_row(U s, int nbrOrbitals, const
           for (int v = 0; v < K; ++v) pend[v] = xr[v];
           pendCoef = coef;
         } else {
-          dh_gather_fma<K>(acc, xbase, idx, coef);
+          dh_gather_fma<K, K == 16>(acc, xbase, idx, coef);
         }
       };
       if constexpr (FREE) {
