@@ -221,7 +221,6 @@ struct dh_sector_set {
   size_t coefCap = 0;
 };
 
-// work descriptor of the active sectors (dh_multisector.hip)
 // tiled spin-1/2 product (dh_spin_tile.hip): its tables, whether it takes blocks of k, the product
 size_t dh_spin_tile_bytes();
 int dh_spin_tile_tables(dh_basis* b);
@@ -229,6 +228,8 @@ bool dh_spin_tiles(const dh_hamiltonian* h, bool uniform, int k);
 int dh_spin_tile_hv(dh_hamiltonian* h, bool uniform, const double* x, double* y, int k, int add, int64_t first,
                     int64_t count);
 
+// the sectors of one product (active == nullptr: all) and their rows; their work descriptor (dh_multisector.hip)
+int64_t dh_sectors_active_rows(const dh_sector_set* S, const unsigned char* active, int* nActive);
 int dh_sectors_upload_work(dh_sector_set* S, const unsigned char* active, int64_t rowsPerTile, int* nActive,
                            int64_t* totalTiles);
 // complex product over a momentum set and its matrix elements per sector (dh_lattice.hip)

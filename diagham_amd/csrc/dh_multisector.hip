@@ -269,6 +269,17 @@ extern "C" int dh_sector_set_blas_launch(dh_sector_set* S, int axpyGroupsPerCU, 
 
 // work descriptor of the active sectors for tiles of `rowsPerTile` rows:
 // d_work[0..na) = sector ids, d_work[na..2na] = tile prefix
+int64_t dh_sectors_active_rows(const dh_sector_set* S, const unsigned char* active, int* nActive) {
+  int64_t rows = 0;
+  *nActive = 0;
+  for (int s = 0; s < S->nbrSectors; ++s) {
+    if (active && !active[s]) continue;
+    rows += S->offsets[s + 1] - S->offsets[s];
+    ++*nActive;
+  }
+  return rows;
+}
+
 int dh_sectors_upload_work(dh_sector_set* S, const unsigned char* active, int64_t rowsPerTile, int* nActive,
                        int64_t* totalTiles) {
   dh_context* c = S->ctx;
@@ -506,43 +517,82 @@ static int sectors_hv_launch(dh_sector_set* S, int blockSize, bool freePairs, co
   return S->triangles ? where(std::true_type{}) : where(std::false_type{});
 }
 
-// Lanes per row, workgroup size and row routine by rows per CU and k, times in us on MI355X.  Few rows: eight
-// lanes and the range loop, whose rows finish together (4173 rows: 14.7, 15.7 with 2 x 256 and the masks; k = 4
-// 16.8 and 17.8).  Then lanes for wavefronts (26 k rows: 19.3 with 2 x 256, 21.5 with 1 x 256; k = 16 43.5 with
-// 4 x 256, 49.9 with 2).  From 128 to 2048 rows a CU small workgroups spread best (164 k rows: 35.4 with
-// 1 x 256, 40 with 1 x 512 and 1 x 1024; k = 4: 55 with 2 x 256, 60 with 1 x 512, 71 by ranges; k = 8: 99, 125
-// by ranges; k = 16: 285 with 4 x 256, 375 with 2 x 512 by ranges).  Above, the tables in LDS bound the
+// What a launch shape costs the sectors of a product, in passes of one wavefront over its rows, from the
+// workgroups that fit a CU and the rounds that the tiles take: up to 16 wavefronts a CU run together, more share
+// its units; a second lane saves 30 % of a pass; with the high rank table in L2 a pass takes 15 % longer.
+// Ranks 190 measured products of 30 k to 500 k rows within 8 % of their fastest shape on average.
+static double sectors_rounds(const dh_sector_set* S, const unsigned char* active, int na, int lanes, int bs) {
+  int tables;
+  const size_t lds = sectors_lds(S, na, bs, &tables);
+  const int64_t cus = S->ctx->nbrCU, fit = std::max<int64_t>(1, std::min<int64_t>(160 * 1024 / lds, 2048 / bs));
+  int64_t tiles = 0;
+  for (int s = 0; s < S->nbrSectors; ++s)
+    if (!active || active[s]) tiles += ((S->offsets[s + 1] - S->offsets[s]) * lanes + bs - 1) >> __builtin_ctz(bs);
+  auto pass = [&](int64_t groups) { return std::max(1.0, groups * (bs / 64) / 16.0); };
+  const int64_t full = tiles / (cus * fit), rest = tiles - full * cus * fit;
+  const double rounds = full * pass(fit) + (rest ? pass((rest + cus - 1) / cus) : 0.0);
+  return rounds * (lanes == 1 ? 1.0 : 0.7) * (tables == 2 ? 1.0 : 1.15);
+}
+
+// Lanes per row, workgroup size and row routine by rows per CU, k and the bytes of the staged tables, times in us on
+// MI355X.  Few rows: eight lanes and the range loop, whose rows finish together (4173 rows: 14.7, 15.7 with 2 x
+// 256 and the masks; k = 4 16.8 and 17.8); large tables are staged by 512 threads, as for a single space (1300
+// rows on 26 orbitals 15.2, 18.7 with 256; k = 8, 7680 rows 20.4, 24.2).  Then lanes for wavefronts (26 k rows:
+// 19.3 with 2 x 256, 21.5 with 1 x 256; k = 16 43.5 with 4 x 256, 49.9 with 2).  From 128 to 2048 rows a CU small
+// workgroups spread best (164 k rows: 35.4 with 1 x 256, 40 with 1 x 512 and 1 x 1024; k = 4: 55 with 2 x 256, 60
+// with 1 x 512, 71 by ranges; k = 8: 99, 125 by ranges; k = 16: 285 with 4 x 256, 375 with 2 x 512 by ranges).
+// Where three of them at most fit a CU, one of another shape that sectors_rounds puts 25 % below is taken (246 k
+// rows on 28 orbitals 71.7 with 1 x 1024, 134 with 1 x 256, k = 4 143 and 238; 329 k rows on 26 67 and 85; for
+// k = 8 only from 900 rows a CU, 192 k rows 127 with 2 x 256 and 137 with 2 x 1024).
+// Above, the tables in LDS bound the
 // wavefronts of a CU: 1024 threads (1.0 M rows: 188, 232 at 256; 17.6 M rows with 29 orbitals: 5.4 ms, 8.4 at
 // 512, 14.0 at 256), 512 once x outgrows the 256 MB behind the L2s and the gathers go to HBM (278 M rows: 191
 // ms, 211 at 1024), for k = 4 512 when three workgroups fit (1.0 M rows, 25 orbitals: 314, 336 at 1024, 425 by
-// ranges).  k = 8: two lanes, 1024 threads where one workgroup's tables fill a CU (6.7 M rows: 6.0 ms, 7.0 with
+// ranges), and with both rank tables in L2 two lanes (1.7 M rows on 39 orbitals 706, 892 with one; k = 4 988
+// and 1073).  k = 8: two lanes, 1024 threads where one workgroup's tables fill a CU (6.7 M rows: 6.0 ms, 7.0 with
 // 2 x 512), 512 where more fit (1.0 M rows: 676, 725 at 1024), one lane with the high table in L2 (17.6 M rows
 // 22.3 ms, 23.7 with two).  k = 16: two lanes, 512, and by ranges (2139, 2242 with the masks).
-static void sectors_shape(const dh_sector_set* S, int k, int* lpr, int* bs, bool* freePairs) {
+//
+// The rows are those of the product's sectors: late in a batched solve few of them are still active (one sector
+// of the set of 7 on 37 orbitals, 20 k of 5.2 M rows: 34 us, 98 with the set's shape).
+static void sectors_shape(const dh_sector_set* S, int k, const unsigned char* active, int* lpr, int* bs,
+                          bool* freePairs) {
   *lpr = S->lanesPerRow;
   *bs = S->blockSize;
   // DH_INDEX_RANK in a chosen shape: the free-pair masks for k <= 2, as for a single space
   *freePairs = S->rowMode == DH_INDEX_RANK_FREE || (S->rowMode == DH_INDEX_RANK && k <= 2);
   if (!S->autoLaunch) return;
-  const int64_t perCU = S->totalDim / S->ctx->nbrCU;
+  int na, tables;
+  const int64_t rows = dh_sectors_active_rows(S, active, &na), perCU = rows / S->ctx->nbrCU;
+  const size_t staged = sectors_lds(S, na, 256, &tables);
   bool masks = true;
   auto set = [&](int l, int b) { *lpr = l, *bs = b; };
   if (perCU < 32) {
-    set(8, 256);
+    set(8, k <= 4 ? (staged > 16 * 1024 ? 512 : 256) : k == 8 && tables && staged > 40 * 1024 ? 512 : 256);
     masks = false;
   } else if (perCU < 128) {
     set(k == 16 ? 4 : 2, 256);
   } else if (perCU < 2048) {
     set(k <= 2 ? 1 : k == 16 ? 4 : 2, 256);
+    if (tables && staged > 40 * 1024 && (k <= 4 || (k == 8 && perCU >= 900))) {
+      const double small = sectors_rounds(S, active, na, *lpr, 256);
+      double best = small / 1.25;
+      for (int l = k == 8 ? 2 : 1; l <= 2; ++l)
+        for (int b = 256; b <= 1024; b *= 2) {
+          const double t = sectors_rounds(S, active, na, l, b);
+          if (t <= best) best = t, set(l, b);
+        }
+    }
   } else if (k == 16) {
     set(2, 512);
     masks = false;
+  } else if (!tables && k <= 4) {
+    set(2, 1024);
   } else {
-    int tables;
-    const bool three = 3 * sectors_lds(S, S->nbrSectors, 512, &tables) <= 160 * 1024;
-    const bool oneFills = sectors_lds(S, S->nbrSectors, 1024, &tables) > 79 * 1024 && tables == 2;
+    const bool three = 3 * sectors_lds(S, na, 512, &tables) <= 160 * 1024;
+    const bool oneFills = sectors_lds(S, na, 1024, &tables) > 79 * 1024 && tables == 2;
     if (k <= 2)
-      set(1, S->totalDim * k <= (int64_t)1 << 25 ? 1024 : 512);
+      set(1, rows * k <= (int64_t)1 << 25 ? 1024 : 512);
     else if (k == 4)
       set(1, three && !oneFills ? 512 : 1024);
     else
@@ -555,7 +605,7 @@ template <int K>
 static int sectors_hv_lpr(dh_sector_set* S, const double* x, double* y, int add, const unsigned char* active) {
   int lpr, bs;
   bool freePairs;
-  sectors_shape(S, K, &lpr, &bs, &freePairs);
+  sectors_shape(S, K, active, &lpr, &bs, &freePairs);
   switch (lpr) {
     case 1: return sectors_hv_launch<K, 1>(S, bs, freePairs, x, y, add, active);
     case 2: return sectors_hv_launch<K, 2>(S, bs, freePairs, x, y, add, active);

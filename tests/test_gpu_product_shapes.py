@@ -67,3 +67,36 @@ def test_small_spaces_in_their_own_shape(arch, n, total_lz, lz_max, k):
         y[j] = c @ X[t]
     for v in range(k):
         assert np.linalg.norm(Y[at][:, v] - y[:, v]) <= 1e-12 * np.linalg.norm(y[:, v]), v
+
+
+# every branch of the rule of sphere sets by rows per CU: few (with small and large tables), below 128, 128 to 2048 with
+# workgroups that fit a CU many times and three times, above 2048 with both rank tables in LDS, one and none; 26 to
+# 28 orbitals restage the high table from sector to sector
+@pytest.mark.parametrize("n,lz_max,step", [(5, 13, 1), (3, 25, 1), (5, 23, 1), (7, 20, 1), (7, 25, 1), (6, 31, 1),
+                                           (8, 24, 1), (7, 27, 1), (6, 35, 1)])
+@pytest.mark.parametrize("k", [1, 2, 4, 8, 16])
+def test_sphere_sets_in_their_own_shape(arch, n, lz_max, step, k):
+    from diagham_amd import capi
+    sectors = capi.sphere_sectors(n, lz_max)
+    V = coulomb(lz_max)
+    S = SectorSet(arch, n, lz_max, sectors, V)
+    fac = O.Factors(lz_max, V)
+    X = np.random.default_rng(lz_max + k).standard_normal((S.total, k))
+    Y = S.hv(X.reshape(-1), k).reshape(S.total, k)
+    active = np.zeros(len(sectors), np.uint8)
+    active[[0, len(sectors) // 2, -1]] = 1
+    Z = S.hv(X.reshape(-1), k, active, Y.reshape(-1).copy()).reshape(S.total, k)
+    for i in sorted({0, 1, len(sectors) // 2, len(sectors) - 1}):
+        ref = O.FermionSphere(n, sectors[i], lz_max)
+        a, b = int(S.off[i]), int(S.off[i + 1])
+        at = np.unique(np.linspace(0, ref.dim - 1, 60).astype(int))
+        y = np.zeros((at.size, k))
+        for j, r in enumerate(at):
+            t, c = O.fs_row_elements(ref, fac, int(r))
+            y[j] = c @ X[a:b][t]
+        for v in range(k):
+            for got in (Y, Z):  # all sectors, and three of them (the rest keep what was there)
+                assert np.linalg.norm(got[a:b][at][:, v] - y[:, v]) <= 1e-12 * np.linalg.norm(y[:, v]), (i, k, v)
+    keep = np.repeat(active == 0, np.diff(S.off))
+    assert np.array_equal(Y[keep], Z[keep])
+    S.close()
