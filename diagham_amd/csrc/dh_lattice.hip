@@ -736,29 +736,68 @@ static int lattice_launch(dh_sector_set* S, int blockSize, const double* x, doub
                : launch(lattice_hv_kernel<K, LPR, false, 64, false>);
 }
 
+// What a launch shape costs the sectors of a product, as sectors_rounds (dh_multisector.hip): 10 wavefronts a CU run
+// together here and 16 fit by their registers, each doubling of the lanes saves 40 % of a pass, and the factors in
+// LDS 15 %.  Ranks 130 measured products of 8 k to 500 k rows and two to eight vectors within 5 % of their fastest
+// shape on average (the shapes below alone: 12 %).
+static double lattice_rounds(const dh_sector_set* S, const unsigned char* active, const LatticeLds& l, int lanes, int bs) {
+  const bool factors = l.factorsFit && bs == 1024;
+  const size_t lds = factors ? l.withFactors : S->d_rankLo16 && l.withLo <= 79 * 1024 ? l.withLo : l.tables;
+  const int64_t cus = S->ctx->nbrCU, fit = std::max<int64_t>(1, std::min<int64_t>(160 * 1024 / lds, 1024 / bs));
+  int64_t tiles = 0;
+  for (int s = 0; s < S->nbrSectors; ++s)
+    if (!active || active[s]) tiles += ((S->offsets[s + 1] - S->offsets[s]) * lanes + bs - 1) >> __builtin_ctz(bs);
+  auto pass = [&](int64_t groups) { return std::max(1.0, groups * (bs / 64) / 10.0); };
+  const int64_t full = tiles / (cus * fit), rest = tiles - full * cus * fit;
+  const double rounds = full * pass(fit) + (rest ? pass((rest + cus - 1) / cus) : 0.0);
+  return rounds * (0.2 + 0.8 / lanes) * (factors ? 0.85 : 1.0);
+}
+
 // Lanes per row and workgroup size by rows per CU and k, times in us on MI355X.  Few rows: lanes for
 // wavefronts (8008 rows: 21.0 with 4 x 256, 25.5 with 1 x 256; k = 4: 24.7 with 8 x 256, 40.8).  Up to
 // 512 rows a CU 2 x 512 (53 k rows: 27.0 against 34.9).  Above, where the factors fit LDS, 1 x 1024
 // with them there (177 k rows 50.9 against 63.3 at 1 x 256 and 60.9 at 2 x 512; 30 M rows 23.5 ms
 // against 31.1 and 29.7); for k > 2 the rows' own gathers weigh more and the line is at 2048 rows a CU
 // (177 k rows, k = 8: 355 at 1 x 256, 392 and more at 1 x 1024; 735 k rows, k = 4: 986 against 639).  Where they don't
-// fit, two lanes (1.9 M rows on 36 sites: 1698 at 2 x 512 against 1882; k = 4: 3509 at 2 x 256, 3856).
-static void lattice_shape(const dh_sector_set* S, int k, int* lpr, int* bs) {
+// fit, two lanes (1.9 M rows on 36 sites: 1698 at 2 x 512 against 1882; k = 4: 3509 at 2 x 256, 3856), and for one
+// vector, where the low rank table is not in LDS either (35 sites and more), four from 800 to 6000 rows a CU (212 k
+// rows on 49 sites 185, 251 with 2 x 512; 658 k on 40 528 and 613; 1.6 M on 35 1323 and 1365).  Up to 2048 rows a
+// CU how the tiles fall on the CUs decides, and a shape that lattice_rounds puts enough below is taken for more
+// than one vector (28 k rows on 32 sites, k = 4: 50 with 4 x 512, 82 with 8 x 256; 194 k on 48 sites, k = 8: 424
+// with 4 x 256, 551 with 2 x 256; 204 k on 30 sites, k = 4: 214 with 1 x 1024, 282 with 1 x 256).
+// The rows are those of the product's sectors (one of 30 sectors of 6 fermions on 6 x 5 sites, 20 k rows, k = 8:
+// 84 us, 558 with the shape of all 594 k).
+static void lattice_shape(const dh_sector_set* S, int k, const unsigned char* active, int* lpr, int* bs) {
   *lpr = S->lanesPerRow;
   *bs = S->blockSize;
   if (!S->autoLaunch) return;
-  const int64_t perCU = S->totalDim / S->ctx->nbrCU;
+  int na;
+  const int64_t perCU = dh_sectors_active_rows(S, active, &na) / S->ctx->nbrCU;
+  const LatticeLds l = lattice_lds(S, na);
   auto set = [&](int l, int b) { *lpr = l, *bs = b; };
-  if (perCU < 128) return k <= 2 ? set(4, 256) : set(8, 256);
-  if (perCU < 512 && k <= 2) return set(2, 512);
-  if (lattice_lds(S, S->nbrSectors).factorsFit) return k > 2 && perCU < 2048 ? set(1, 256) : set(1, 1024);
-  k <= 2 ? set(2, 512) : set(2, 256);
+  if (perCU < 128)
+    set(k <= 2 ? 4 : 8, 256);
+  else if (perCU < 512 && k <= 2)
+    set(2, 512);
+  else if (l.factorsFit)
+    k > 2 && perCU < 2048 ? set(1, 256) : set(1, 1024);
+  else if (k == 1 && !S->d_rankLo16 && perCU >= 800 && perCU < 6000)
+    set(4, 512);
+  else
+    k <= 2 ? set(2, 512) : set(2, 256);
+  if (k == 1 || perCU < (k == 2 ? 128 : 32) || perCU >= 2048) return;
+  double best = lattice_rounds(S, active, l, *lpr, *bs) / (k == 2 ? 1.25 : 1.15);
+  for (int lanes = 1; lanes <= 8; lanes *= 2)
+    for (int b = 256; b <= 1024; b *= 2) {
+      const double t = lattice_rounds(S, active, l, lanes, b);
+      if (t <= best) best = t, set(lanes, b);
+    }
 }
 
 template <int K>
 static int lattice_lpr(dh_sector_set* S, const double* x, double* y, int add, const unsigned char* active) {
   int lpr, bs;
-  lattice_shape(S, K, &lpr, &bs);
+  lattice_shape(S, K, active, &lpr, &bs);
   switch (lpr) {
     case 1: return lattice_launch<K, 1>(S, bs, x, y, add, active);
     case 2: return lattice_launch<K, 2>(S, bs, x, y, add, active);

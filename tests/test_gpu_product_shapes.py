@@ -100,3 +100,36 @@ def test_sphere_sets_in_their_own_shape(arch, n, lz_max, step, k):
     keep = np.repeat(active == 0, np.diff(S.off))
     assert np.array_equal(Y[keep], Z[keep])
     S.close()
+
+
+# the same for momentum sets: factors in LDS or not, the low rank table in LDS or not (35 sites and more)
+@pytest.mark.parametrize("n,nx,ny", [(4, 4, 4), (5, 5, 4), (5, 6, 4), (6, 6, 5), (5, 8, 4), (4, 6, 6), (5, 7, 5), (4, 8, 6)])
+@pytest.mark.parametrize("k", [1, 2, 4, 8])
+def test_momentum_sets_in_their_own_shape(arch, n, nx, ny, k):
+    from test_gpu_lattice import T1, T2, TPP, MomentumSet
+    sectors = [(x, y) for x in range(nx) for y in range(ny)]
+    S = MomentumSet(arch, n, nx, ny, sectors)
+    c = S.capi
+    u, _ = O.checkerboard_lower_band(nx, ny, T1, T2, TPP)
+    fac = O.LatticeFactors(nx, ny, u)
+    rng = np.random.default_rng(n + k)
+    X = rng.standard_normal((S.total, k)) + 1j * rng.standard_normal((S.total, k))
+    Y = S.hv(X, k)
+    active = np.zeros(len(sectors), np.uint8)
+    active[[0, len(sectors) // 2]] = 1
+    dx = c.DeviceBuffer.from_host(arch, np.ascontiguousarray(X).view(np.float64).reshape(-1))
+    dz = c.DeviceBuffer(arch, 2 * S.total * k)
+    arch.check(c.gpu().dh_sectors_hv(S.h, dx.ptr, dz.ptr, k, 0, bytes(active)), "hv")
+    Z = dz.download().view(np.complex128).reshape(S.total, k)
+    for i in (0, len(sectors) // 2):
+        ref = O.MomentumFermions(n, nx, ny, *sectors[i])
+        a, b = int(S.off[i]), int(S.off[i + 1])
+        at = np.unique(np.linspace(0, ref.dim - 1, 40).astype(int))
+        y = np.zeros((at.size, k), complex)
+        for j, r in enumerate(at):
+            t, coef = O.fm_row_elements(ref, fac, int(r))
+            y[j] = coef.conj() @ X[a:b][t]  # listed by source state: H[t, r]
+        for v in range(k):
+            for got in (Y, Z):
+                assert np.linalg.norm(got[a:b][at][:, v] - y[:, v]) <= 1e-12 * np.linalg.norm(y[:, v]), (i, k, v)
+    S.close()
