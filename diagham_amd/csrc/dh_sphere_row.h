@@ -12,8 +12,6 @@
 // (half the instructions for every shift, mask, ctz and popcount of the row routine).
 __device__ __forceinline__ int dh_ctz(uint64_t v) { return __builtin_ctzll(v); }
 __device__ __forceinline__ int dh_ctz(uint32_t v) { return __builtin_ctz(v); }
-__device__ __forceinline__ int dh_popc(uint64_t v) { return __popcll(v); }
-__device__ __forceinline__ int dh_popc(uint32_t v) { return __popc(v); }
 
 // Off-diagonal factors of annihilated pair i of one sum in LDS (dh_pack_sphere_factors): a square's row,
 // or one triangle.  The entry of sBase packs where the sum's table starts and its number of pairs.
@@ -62,8 +60,8 @@ __device__ __forceinline__ void dh_gather_fma(double* acc, const double* __restr
   }
 }
 
-__device__ __forceinline__ uint64_t dh_bitrev(uint64_t v) { return __builtin_bitreverse64(v); }
-__device__ __forceinline__ uint32_t dh_bitrev(uint32_t v) { return __builtin_bitreverse32(v); }
+__host__ __device__ __forceinline__ uint64_t dh_bitrev(uint64_t v) { return __builtin_bitreverse64(v); }
+__host__ __device__ __forceinline__ uint32_t dh_bitrev(uint32_t v) { return __builtin_bitreverse32(v); }
 
 // What a row state s tells about the pairs (m3 > m4) of one orbital sum S, as 32-bit masks over their
 // positions i = m3 - lo(S), m3 = lo(S) + i, m4 = m4hi(S) - i, lo(S) = S/2 + 1, m4hi(S) = (S - 1)/2
@@ -83,7 +81,7 @@ template <typename U>
 struct dh_row_masks {
   static constexpr int W = 8 * sizeof(U);
   U f, rf, par, rpar;
-  __device__ __forceinline__ dh_row_masks(U s, int nbrOrbitals) {
+  __host__ __device__ __forceinline__ dh_row_masks(U s, int nbrOrbitals) {
     const U full = nbrOrbitals >= W ? ~U(0) : ((U(1) << nbrOrbitals) - U(1));
     f = ~s & full;
     rf = dh_bitrev(f);
@@ -92,10 +90,10 @@ struct dh_row_masks {
     for (int o = 1; o < W; o <<= 1) par ^= par << o;
     rpar = dh_bitrev(par);
   }
-  __device__ __forceinline__ uint32_t free(int m3lo, int m4hi) const {
+  __host__ __device__ __forceinline__ uint32_t free(int m3lo, int m4hi) const {
     return (uint32_t)(f >> m3lo) & (uint32_t)(rf >> (W - 1 - m4hi));
   }
-  __device__ __forceinline__ uint32_t sign(int m3lo, int m4hi) const {
+  __host__ __device__ __forceinline__ uint32_t sign(int m3lo, int m4hi) const {
     return (uint32_t)(par >> m3lo) ^ (uint32_t)(rpar >> (W - 1 - m4hi));
   }
 };

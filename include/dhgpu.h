@@ -211,7 +211,7 @@ int dh_sector_set_get_states(dh_sector_set* set, uint64_t* states);
 int dh_sector_set_factors(dh_sector_set* set, const double* factors, const int* pair_offset, int nbr_factors,
                           double shift);
 /* Launch shape of the set's products.  Until it is called, sphere and momentum sets pick their shape
- * per product from k and their rows per CU. */
+ * per product from k, the rows per CU of its active sectors and the tables that a workgroup stages. */
 int dh_sector_set_launch(dh_sector_set* set, int lanes_per_row, int block_size);
 /* Row routine of the products of a sphere or momentum set: DH_INDEX_RANK_RANGE (every created pair
  * of the range or list, skipping occupied ones), DH_INDEX_RANK_FREE (only the free created pairs,

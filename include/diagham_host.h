@@ -124,7 +124,10 @@ int dhh_sectors_alone_rows(int64_t rows);
  * sectors to nbr_eigen eigenvalues with that shape.  The block size whose calibration solve is
  * shortest wins: best = {k, lanes per row, workgroup, row mode}.  table: 7 doubles per ks[i]: k,
  * lanes per row, workgroup, row mode, product ms, calibration seconds (-1: the vectors did not fit),
- * vector products of the calibration solve.  Apply the result with dhh_sectors_launch. */
+ * vector products of the calibration solve.  Apply the result with dhh_sectors_launch.  The shapes that
+ * the sets choose by themselves (dhh_sectors_launch with lanes_per_row = 0), by k and the rows of each
+ * product, are not among the candidates, and have workgroups of 512 and rows on 8 lanes besides: they
+ * can be the faster ones. */
 int dhh_sectors_autotune(dhh_arch* arch, int nbr_fermions, int lz_max, const int* total_lz, int nbr_sectors,
                          const double* pseudopotentials, int nbr_eigen, const int* ks, int nbr_ks, double fraction,
                          int max_iter, uint64_t seed, double* table, int* best);

@@ -46,10 +46,23 @@ def test_sector_rows_on_one_lane_of_64_bit_words(arch, n, lz_max, sectors, k, ro
     S.close()
 
 
+# rank tables in LDS (26 to 28 orbitals, restaged from sector to sector; 29 never) in chosen shapes
+@pytest.mark.parametrize("n,lz_max,lpr,block", [(4, 25, 1, 256), (4, 26, 2, 1024), (4, 27, 1, 1024), (4, 27, 1, 512),
+                                                (4, 28, 1, 1024)])
+@pytest.mark.parametrize("k", [2, 4, 16])
+def test_every_column_with_rank_tables_in_lds(arch, n, lz_max, lpr, block, k):
+    sectors = list(range((n * lz_max) % 2, 60, 2))
+    V = coulomb(lz_max)
+    S = SectorSet(arch, n, lz_max, sectors, V)
+    assert S.capi.gpu().dh_sector_set_launch(S.h, lpr, block) == 0
+    sphere_set_matches(S, n, lz_max, sectors, V, k, rows=40)
+    S.close()
+
+
 # a space in every branch of the rule below 256 rows per CU: few rows with small and large tables, from 64 and from
-# 128 rows per CU, with the low rank table in LDS and in global memory
+# 128 rows per CU, with the low rank table in LDS and in global memory; and one whose rank tables are both in LDS
 @pytest.mark.parametrize("n,total_lz,lz_max", [(6, 0, 15), (3, 0, 26), (5, 0, 36), (6, 1, 31), (5, 0, 44), (7, 0, 30),
-                                               (6, 0, 40)])
+                                               (6, 0, 40), (10, 0, 27)])
 @pytest.mark.parametrize("k", [1, 4, 8, 16])
 def test_small_spaces_in_their_own_shape(arch, n, total_lz, lz_max, k):
     from diagham_amd import capi
