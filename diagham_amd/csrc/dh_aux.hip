@@ -442,7 +442,7 @@ __global__ void __launch_bounds__(kAdjointThreads) sphere_adjoint_kernel(int nbr
             pm &= pm - 1;
             const U w = t | (U(1) << (m3lo + i)) | (U(1) << (m4hi - i));
             constexpr bool FAR = dh_far_tables<U, false>;
-            idx[q] = dh_rank_of<FAR>(w, dh_entry<FAR>(lo, (uint32_t)(w & loMask)), hi, rankBits, last);
+            idx[q] = dh_rank_of<FAR>(w, [&] { return dh_entry<FAR>(lo, (uint32_t)(w & loMask)); }, hi, rankBits, last);
             pos[q] = i;
           }
         }

@@ -164,7 +164,7 @@ __global__ void __launch_bounds__(1024) sphere_hv_kernel(SphereArgs a, const dou
     if constexpr (WORDS == 1 && BASE != MODE_BSEARCH) {
       const uint32_t last = (uint32_t)a.dim - 1u, mask = (1u << a.rankBits) - 1u;
       const int bits = a.rankBits;
-      auto find = [&](uint32_t t) -> uint32_t { return dh_rank_of<false>(t, loAt(t & mask), sHi, bits, last); };
+      auto find = [&](uint32_t t) -> uint32_t { return dh_rank_of<false>(t, [&] { return loAt(t & mask); }, sHi, bits, last); };
       if constexpr (ROW == ROW_X4)
         diag = dh_sphere_row_x4<K, LPR, TRI>((uint32_t)s, a.nbrOrbitals, sF, sBase, lane, find, x, acc);
       else
@@ -175,7 +175,8 @@ __global__ void __launch_bounds__(1024) sphere_hv_kernel(SphereArgs a, const dou
       const uint32_t mask = a.rankBits >= 32 ? 0xffffffffu : (1u << a.rankBits) - 1u;
       const int bits = a.rankBits;
       auto find = [&](uint64_t t) -> uint32_t {
-        return dh_rank_of<dh_far_tables<uint64_t, BASE != MODE_RANK_GLOBAL>>(t, loAt((uint32_t)t & mask), sHi, bits, last);
+        return dh_rank_of<dh_far_tables<uint64_t, BASE != MODE_RANK_GLOBAL>>(
+            t, [&] { return loAt((uint32_t)t & mask); }, sHi, bits, last);
       };
       if constexpr (ROW == ROW_X4)
         diag = dh_sphere_row_x4<K, LPR, TRI>(s, a.nbrOrbitals, sF, sBase, lane, find, x, acc);

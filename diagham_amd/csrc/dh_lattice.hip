@@ -551,7 +551,8 @@ __global__ void __launch_bounds__(1024) lattice_hv_kernel(LatticeArgs a, const d
       const uint32_t last = (uint32_t)dim - 1u, mask = (uint32_t)a.loSize - 1u;
       const int bits = a.rankBits;
       auto find = [&](U t) -> uint32_t {
-        return dh_rank_of<dh_far_tables<U, LO_LDS>>(t, lo[(uint32_t)t & mask], hi, bits, last);
+        return dh_rank_of<dh_far_tables<U, LO_LDS>>(
+            t, [&] { return (uint32_t)lo[(uint32_t)t & mask]; }, hi, bits, last);
       };
       const double2* fac;
       if constexpr (FAC_LDS)

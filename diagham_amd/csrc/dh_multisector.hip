@@ -403,7 +403,7 @@ __global__ void __launch_bounds__(1024) sectors_hv_kernel(SectorsArgs a, const d
     if constexpr (S32) {
       const uint32_t last = (uint32_t)dim - 1u, mask = (1u << a.rankBits) - 1u;
       const int bits = a.rankBits;
-      auto find = [&](uint32_t t) -> uint32_t { return dh_rank_of<false>(t, loAt(t & mask), hi, bits, last); };
+      auto find = [&](uint32_t t) -> uint32_t { return dh_rank_of<false>(t, [&] { return loAt(t & mask); }, hi, bits, last); };
       diag = dh_sphere_row<K, LPR, FREE, TRI>((uint32_t)s, a.nbrOrbitals, sF, sBase, lane, find, x + off * K, acc);
     } else {
       // rankBits = ceil(orbitals / 2) <= 32, so t >> bits fits 32 bits
@@ -411,7 +411,8 @@ __global__ void __launch_bounds__(1024) sectors_hv_kernel(SectorsArgs a, const d
       const uint32_t mask = a.rankBits >= 32 ? 0xffffffffu : (1u << a.rankBits) - 1u;
       const int bits = a.rankBits;
       auto find = [&](uint64_t t) -> uint32_t {
-        return dh_rank_of<dh_far_tables<uint64_t, (TABLES > 0)>>(t, loAt((uint32_t)t & mask), hi, bits, last);
+        return dh_rank_of<dh_far_tables<uint64_t, (TABLES > 0)>>(
+            t, [&] { return loAt((uint32_t)t & mask); }, hi, bits, last);
       };
       diag = dh_sphere_row<K, LPR, FREE, TRI>(s, a.nbrOrbitals, sF, sBase, lane, find, x + off * K, acc);
     }

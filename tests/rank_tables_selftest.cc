@@ -27,8 +27,8 @@ static int check(int orbitals, uint32_t* lo, uint32_t* hi) {
     lo[state & loMask] = 17;
     const U t = (U)state;
     const uint32_t l = dh_entry<FAR>(lo, (uint32_t)(t & (U)loMask));
-    wrong += dh_rank_of<FAR>(t, l, hi, bits, 5000u) != 983u;
-    wrong += dh_rank_of<FAR>(t, l, hi, bits, 400u) != 400u;  // clamped
+    wrong += dh_rank_of<FAR>(t, [&] { return l; }, hi, bits, 5000u) != 983u;
+    wrong += dh_rank_of<FAR>(t, [&] { return l; }, hi, bits, 400u) != 400u;  // clamped
     hi[state >> bits] = 0;
     lo[state & loMask] = 0;
   }
