@@ -759,7 +759,8 @@ static double lattice_rounds(const dh_sector_set* S, const unsigned char* active
 // 512 rows a CU 2 x 512 (53 k rows: 27.0 against 34.9).  Above, where the factors fit LDS, 1 x 1024
 // with them there (177 k rows 50.9 against 63.3 at 1 x 256 and 60.9 at 2 x 512; 30 M rows 23.5 ms
 // against 31.1 and 29.7); for k > 2 the rows' own gathers weigh more and the line is at 2048 rows a CU
-// (177 k rows, k = 8: 355 at 1 x 256, 392 and more at 1 x 1024; 735 k rows, k = 4: 986 against 639).  Where they don't
+// (177 k rows, k = 8: 355 at 1 x 256, 392 and more at 1 x 1024; 735 k rows, k = 4: 986 against 639), at 1280 with the
+// high rank table there too (346 k rows on 25 sites, k = 4: 559 and 483, k = 8 1407 and 1281).  Where they don't
 // fit, two lanes (1.9 M rows on 36 sites: 1698 at 2 x 512 against 1882; k = 4: 3509 at 2 x 256, 3856), and for one
 // vector, where the low rank table is not in LDS either (35 sites and more), four from 800 to 6000 rows a CU (212 k
 // rows on 49 sites 185, 251 with 2 x 512; 658 k on 40 528 and 613; 1.6 M on 35 1323 and 1365).  Up to 2048 rows a
@@ -781,14 +782,16 @@ static void lattice_shape(const dh_sector_set* S, int k, const unsigned char* ac
   else if (perCU < 512 && k <= 2)
     set(2, 512);
   else if (l.factorsFit)
-    k > 2 && perCU < 2048 ? set(1, 256) : set(1, 1024);
+    k > 2 && perCU < (l.hiFits ? 1280 : 2048) ? set(1, 256) : set(1, 1024);
   else if (k == 1 && !S->d_rankLo16 && perCU >= 800 && perCU < 6000)
     set(4, 512);
   else
     k <= 2 ? set(2, 512) : set(2, 256);
   if (k == 1 || perCU < (k == 2 ? 128 : 32) || perCU >= 2048) return;
   double best = lattice_rounds(S, active, l, *lpr, *bs) / (k == 2 ? 1.25 : 1.15);
-  for (int lanes = 1; lanes <= 8; lanes *= 2)
+  // (over several rounds, blocks without the factors in LDS take longer on one lane than the rounds say: 510 k rows on
+  // 35 sites, k = 4, 942 with 1 x 256, 796 with 2 x 256; 270 k on 36 616 and 543; but 195 k on 48 228 and 277)
+  for (int lanes = k > 2 && !l.factorsFit && perCU >= 1024 ? 2 : 1; lanes <= 8; lanes *= 2)
     for (int b = 256; b <= 1024; b *= 2) {
       const double t = lattice_rounds(S, active, l, lanes, b);
       if (t <= best) best = t, set(lanes, b);
