@@ -444,9 +444,9 @@ __device__ __forceinline__ unsigned dh_xcd_block(unsigned b, unsigned n) {
 // followed by one whole matrix (row i at i * np) for both sums, and a factor is one offset away.  Other
 // tables, and those of more than 100 KiB (52 orbitals), keep one triangle per sum, j (j + 1) / 2 + i for
 // i <= j, with eight more instructions per factor and 7 to 8 % less LDS: on 52 to 58 orbitals both forms take
-// the same time within 3 % (4 fermions on 56: 15.3 us by triangles and 14.8, k = 8 57.7 and 58.0).  An entry of base packs where the sum's matrix starts and its
-// number of pairs.  Input: the per-pair layout (pair a, created m3 from lo(S):
-// factors[pairOffset[a] + m3 - lo(S)]).
+// the same time within 3 % (4 fermions on 56: 15.3 us by triangles and 14.8, k = 8 57.7 and 58.0).  An entry
+// of base packs where the sum's matrix starts and its number of pairs.  Input: the per-pair layout (pair a,
+// created m3 from lo(S): factors[pairOffset[a] + m3 - lo(S)]).
 constexpr int DH_SUM_BASE_BITS = 24;
 constexpr int DH_SUM_BASE_MASK = (1 << DH_SUM_BASE_BITS) - 1;
 

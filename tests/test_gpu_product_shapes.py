@@ -146,3 +146,21 @@ def test_momentum_sets_in_their_own_shape(arch, n, nx, ny, k):
             for got in (Y, Z):
                 assert np.linalg.norm(got[a:b][at][:, v] - y[:, v]) <= 1e-12 * np.linalg.norm(y[:, v]), (i, k, v)
     S.close()
+
+
+# the most orbitals: rank tables of 2^31 words each (built on the host in about 40 s, 8 GiB each), where a byte
+# offset into them does not fit 32 bits
+def test_products_on_62_orbitals(arch):
+    from diagham_amd import capi
+    n, total_lz, lz_max = 3, 1, 61
+    V = coulomb(lz_max)
+    p = capi.Problem.sphere(arch, n, total_lz, lz_max, V)
+    space, fac = O.FermionSphere(n, total_lz, lz_max), O.Factors(lz_max, V)
+    assert p.dim == space.dim
+    for k in (1, 2, 4, 8):
+        X = np.random.default_rng(lz_max + k).standard_normal((p.dim, k))
+        Y = p.hv(X.reshape(-1), k).reshape(p.dim, k)
+        for v in range(k):
+            y = O.fs_hv(space, fac, np.ascontiguousarray(X[:, v]))
+            assert np.linalg.norm(Y[:, v] - y) <= 1e-12 * np.linalg.norm(y), (k, v)
+    p.close()
